@@ -1,0 +1,72 @@
+"""The run-time-geometry variants of the attention kernels: any group up to 16
+query heads per kv head and any head_dim up to 128, against the f64 reference
+(CpuReferenceBackend::decode, portable.rs:575-646).
+
+Bound per output: half a BF16 step of the value (2^-8 |ref|), plus 2^-13 of
+the largest |v|: probabilities enter P.V as two BF16 parts (relative error
+2^-17 of each, and of their sum), scores are f32 sums of exact BF16 products
+(for |score| < 32 an error below 2^-15, so p moves by less than 2^-14).  One
+BF16 part per probability (2^-9) does not fit it.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from _data import from_torch, normal_bf16, to_torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(got_bits, ref, v_bits, label):
+    got = oracle.read_bf16(np.asarray(got_bits, np.uint16).reshape(-1)).astype(np.float64)
+    ref = np.asarray(ref, np.float64).reshape(-1)
+    bound = np.abs(ref) * 2.0 ** -8 + np.abs(oracle.read_bf16(v_bits.reshape(-1))).max() * 2.0 ** -13
+    over = np.abs(got - ref) > bound
+    assert not over.any(), (label, int(over.sum()), float((np.abs(got - ref) / bound).max()))
+
+
+def _unaligned(t):
+    """The same values two bytes past a 16-byte boundary."""
+    room = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    room[1:].copy_(t.reshape(-1))
+    return room[1:].view(t.shape)
+
+
+# (q heads, kv heads, head_dim): groups without a variant of their own, the
+# largest and smallest head_dim of both run-time variants and odd pieces of 8.
+DECODE = [(3, 1, 128), (10, 2, 128), (36, 3, 120), (16, 1, 72), (15, 1, 64), (12, 4, 64), (7, 7, 40), (6, 2, 8)]
+
+
+@pytest.mark.parametrize("qh,kvh,d", DECODE)
+def test_decode_any_group(ctx, qh, kvh, d):
+    rng = np.random.default_rng(qh * 1000 + d)
+    lens = [1, 15, 33, 64, 257, 1025]
+    b, stride = len(lens), max(lens)
+    qb, kb, vb = (normal_bf16(rng, s) for s in ((b, qh, d), (b, stride, kvh, d), (b, stride, kvh, d)))
+    q, k, v = to_torch(qb), to_torch(kb), to_torch(vb)
+    pages = [-(-t // 16) for t in lens]
+    table = np.zeros((b, max(pages)), np.int32)
+    order = rng.permutation(sum(pages)).astype(np.int32)
+    for i, n in enumerate(pages):
+        table[i, :n] = order[sum(pages[:i]):sum(pages[:i]) + n]
+    table = torch.from_numpy(table).cuda()
+    k_pool = torch.zeros((sum(pages), kvh, 16, d), dtype=torch.int16, device="cuda")
+    v_pool = torch.zeros_like(k_pool)
+    for i, t in enumerate(lens):
+        ctx.pages_write(k_pool, v_pool, table[i], 16, kvh, d, 0, t, k[i, :t].contiguous(), v[i, :t].contiguous())
+    ref = [oracle.cpu_reference_decode(oracle.read_bf16(qb[i]), kb[i, :t], vb[i, :t], 1, qh, kvh, d)[1]
+           for i, t in enumerate(lens)]
+    for split in (0, 64):
+        dense, paged, noalloc, plain = (torch.empty_like(q) for _ in range(4))
+        ctx.decode_dense(q, k, v, dense, lens, qh, kvh, d, seq_stride_tokens=stride, split_tokens=split)
+        ctx.decode_paged(q, k_pool, v_pool, paged, lens, table, max(pages), 16, qh, kvh, d, split_tokens=split)
+        ctx.decode_paged_noalloc(q, k_pool, v_pool, noalloc, lens, table, max(pages), 16, qh, kvh, d,
+                                 split_tokens=split)
+        # unaligned queries take the any-geometry kernel
+        ctx.decode_dense(_unaligned(q), k, v, plain, lens, qh, kvh, d, seq_stride_tokens=stride, split_tokens=split)
+        torch.cuda.synchronize()
+        assert torch.equal(dense, paged) and torch.equal(dense, noalloc)
+        for i in range(b):
+            _check(from_torch(dense[i]), ref[i], vb[i], f"split {split} sequence {i}")
+            _check(from_torch(plain[i]), ref[i], vb[i], f"unaligned, split {split} sequence {i}")

@@ -77,7 +77,7 @@ struct DeviceArgs {
     const int32_t *page_table;
     int64_t seq_stride_tokens;
     int pages_per_seq, page_shift;
-    int batch, q_heads, kv_heads;
+    int batch, q_heads, kv_heads, head_dim;
     int split_tokens;
     float scale_log2e;
     // List mode (list_bins > 0, the LIST kernel): workgroup w runs the
@@ -128,24 +128,24 @@ __device__ __forceinline__ Tables tables_of(const DeviceArgs &a) {
 }
 
 // Base of the 16-token block starting at logical token t0 (a multiple of 16).
-template <int D, bool PAGED>
+template <bool PAGED>
 __device__ __forceinline__ const uint16_t *block_base(const DeviceArgs &a, const uint16_t *cache,
-                                                      int b, int kvh, int t0) {
+                                                      int b, int kvh, int t0, int dim) {
     if constexpr (PAGED) {
         const int shift = a.page_shift;
         const int page = a.page_table[(int64_t)b * a.pages_per_seq + (t0 >> shift)];
         const int64_t row = (((int64_t)page * a.kv_heads + kvh) << shift) + (t0 & ((1 << shift) - 1));
-        return cache + row * D;
+        return cache + row * dim;
     } else {
-        return cache + (((int64_t)b * a.seq_stride_tokens + t0) * a.kv_heads + kvh) * D;
+        return cache + (((int64_t)b * a.seq_stride_tokens + t0) * a.kv_heads + kvh) * dim;
     }
 }
 
 // Element stride between consecutive token rows inside a 16-token block.
-template <int D, bool PAGED>
-__device__ __forceinline__ int row_stride(const DeviceArgs &a) {
-    if constexpr (PAGED) return D;
-    else return a.kv_heads * D;
+template <bool PAGED>
+__device__ __forceinline__ int row_stride(const DeviceArgs &a, int dim) {
+    if constexpr (PAGED) return dim;
+    else return a.kv_heads * dim;
 }
 
 // Ordering point for LDS traffic inside one wavefront: a wavefront's LDS
@@ -213,6 +213,22 @@ template <int D, int G>
 __device__ __forceinline__ void merge_splits(const DeviceArgs &a, int b, int kvh, int tid, int nthreads,
                                              bool coherent);
 
+// Group size and head dimension of a kernel variant.  G > 0 fixes both at
+// compile time.  G == 0 takes any group of at most 16 query heads and any
+// head dimension that is a multiple of 8 up to D at run time: the group is
+// the same zero-padded MFMA N tile, and 16-byte pieces of a row past the head
+// dimension are zeros in K.Q^T and never written from P.V.
+template <int G>
+__device__ __forceinline__ int group_of(const DeviceArgs &a) {
+    if constexpr (G > 0) return G;
+    else return a.q_heads / a.kv_heads;
+}
+template <int D, int G>
+__device__ __forceinline__ int dim_of(const DeviceArgs &a) {
+    if constexpr (G > 0) return D;
+    else return a.head_dim;
+}
+
 template <int D, int G, bool PAGED, bool FUSED, bool NT, bool LIST>
 __global__ __launch_bounds__(64 * kWaves, 2) void decode_kernel(DeviceArgs a) {
     constexpr int DEPTH = kDepth;
@@ -223,10 +239,18 @@ __global__ __launch_bounds__(64 * kWaves, 2) void decode_kernel(DeviceArgs a) {
     constexpr int NS = D / 16;        // P.V MFMA output slices of 16 dims
     constexpr int VT = kTile + 8;     // transposed V row (one dim), in elements
     static_assert(G <= 16, "one MFMA N tile covers the GQA group");
+    // The run-time variant keeps P to 16 bits of mantissa, as the sum of two
+    // BF16 parts (one more MFMA per output slice; the launch stays bound by
+    // its K/V stream): the shapes it serves have had f32 probabilities in the
+    // any-geometry kernel, whose error against 64 bits it matches (below).
+    constexpr bool SPLIT_P = G == 0;
+    constexpr int GM = G > 0 ? G : 16;  // heads the LDS arrays hold
+    const int gn = group_of<G>(a);
+    const int dn = dim_of<D, G>(a);
 
     __shared__ __align__(16) uint16_t vt_lds[kWaves][D * VT];
-    __shared__ float comb_ml[kWaves][G][2];
-    __shared__ float comb_acc[kWaves][G][D];
+    __shared__ float comb_ml[kWaves][GM][2];
+    __shared__ float comb_acc[kWaves][GM][D];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -263,9 +287,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void decode_kernel(DeviceArgs a) {
     const int begin = split * a.split_tokens;
     const int end = min(seq_len, begin + a.split_tokens);
     const int ntiles = (end - begin + kTile - 1) / kTile;
-    const int qh0 = kvh * G;
+    const int qh0 = kvh * gn;
     const float c = a.scale_log2e;
-    const int rs = row_stride<D, PAGED>(a);
+    const int rs = row_stride<PAGED>(a, dn);
     uint16_t *vt = vt_lds[wave];
 
     // Q as the B operand of S^T = K.Q^T: lane holds head row16, dims
@@ -273,9 +297,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void decode_kernel(DeviceArgs a) {
     bf16x8_t qf[KS];
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
-        if (row16 < G)
+        if (row16 < gn && (G > 0 || j * 32 + grp * 8 < dn))
             qf[j] = *reinterpret_cast<const bf16x8_t *>(
-                a.q + ((int64_t)b * a.q_heads + qh0 + row16) * D + j * 32 + grp * 8);
+                a.q + ((int64_t)b * a.q_heads + qh0 + row16) * dn + j * 32 + grp * 8);
         else
             qf[j] = bf16x8_t{};
     }
@@ -297,19 +321,22 @@ __global__ __launch_bounds__(64 * kWaves, 2) void decode_kernel(DeviceArgs a) {
         for (int blk = 0; blk < 2; ++blk) {
             const int bt = min(t0 + blk * 16, last & ~15);
             const int row = min(t0 + blk * 16 + row16, last) - bt;
-            const uint16_t *p = block_base<D, PAGED>(a, a.k, b, kvh, bt) + row * rs + grp * 8;
+            const uint16_t *p = block_base<PAGED>(a, a.k, b, kvh, bt, dn) + row * rs;
+            // a piece past a run-time head dimension re-reads the row's last
+            // one: finite or not it is replaced by zeros in compute_tile
 #pragma unroll
-            for (int j = 0; j < KS; ++j) r.k[blk][j] = kv_load8<NT>(p + j * 32);
+            for (int j = 0; j < KS; ++j)
+                r.k[blk][j] = kv_load8<NT>(p + (G > 0 ? j * 32 + grp * 8 : min(j * 32 + grp * 8, dn - 8)));
         }
-        const uint16_t *vb0 = block_base<D, PAGED>(a, a.v, b, kvh, min(t0, last & ~15));
-        const uint16_t *vb1 = block_base<D, PAGED>(a, a.v, b, kvh, min(t0 + 16, last & ~15));
+        const uint16_t *vb0 = block_base<PAGED>(a, a.v, b, kvh, min(t0, last & ~15), dn);
+        const uint16_t *vb1 = block_base<PAGED>(a, a.v, b, kvh, min(t0 + 16, last & ~15), dn);
         const int blk = (vh * NV) >> 4;  // rows of one lane never straddle a block
         const int bt = min(t0 + blk * 16, last & ~15);
         const uint16_t *vb = blk ? vb1 : vb0;
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int row = min(t0 + vh * NV + i, last) - bt;
-            r.v[i] = kv_load4<NT>(vb + row * rs + vc * 8);
+            r.v[i] = kv_load4<NT>(vb + row * rs + (G > 0 ? vc * 8 : min(vc * 8, dn - 8)));
         }
     };
 
@@ -346,8 +373,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void decode_kernel(DeviceArgs a) {
         for (int blk = 0; blk < 2; ++blk) {
             s[blk] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int j = 0; j < KS; ++j)
-                s[blk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r.k[blk][j], qf[j], s[blk], 0, 0, 0);
+            for (int j = 0; j < KS; ++j) {
+                bf16x8_t kf = r.k[blk][j];
+                if (G == 0 && j * 32 + grp * 8 >= dn) kf = bf16x8_t{};
+                s[blk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[j], s[blk], 0, 0, 0);
+            }
         }
         // Lane holds head row16, tokens t0 + blk*16 + grp*4 + i.
         if (t0 + kTile > end) {
@@ -369,15 +399,21 @@ __global__ __launch_bounds__(64 * kWaves, 2) void decode_kernel(DeviceArgs a) {
         // exactly where the S^T accumulator left it.
         // The row sum adds the same BF16-rounded p that the P.V MFMA
         // multiplies, so O / l is a convex combination of V rows.
-        bf16x8_t pa;
+        bf16x8_t pa, pl;  // pl: SPLIT_P only, the rounding error of pa
         float psum = 0.0f;
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const __bf16 p = (__bf16)__builtin_amdgcn_exp2f(fmaf(s[blk][i], c, -mc));
+                const float pf = __builtin_amdgcn_exp2f(fmaf(s[blk][i], c, -mc));
+                const __bf16 p = (__bf16)pf;
                 psum += (float)p;
                 pa[blk * 4 + i] = p;
+                if constexpr (SPLIT_P) {
+                    const __bf16 low = (__bf16)(pf - (float)p);
+                    psum += (float)low;
+                    pl[blk * 4 + i] = low;
+                }
             }
         l_run = l_run * alpha + psum;
         m_run = m_new;
@@ -398,6 +434,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void decode_kernel(DeviceArgs a) {
             const uint2 hi = *reinterpret_cast<const uint2 *>(src + 16);
             const bf16x8_t vb = __builtin_bit_cast(bf16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
             o[sl] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, vb, o[sl], 0, 0, 0);
+            if constexpr (SPLIT_P) o[sl] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, vb, o[sl], 0, 0, 0);
         }
         wave_lds_fence();
     };
@@ -430,26 +467,26 @@ __global__ __launch_bounds__(64 * kWaves, 2) void decode_kernel(DeviceArgs a) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int h = 4 * grp + i;
-        if (h < G) {
+        if (h < gn) {
 #pragma unroll
             for (int sl = 0; sl < NS; ++sl) comb_acc[wave][h][sl * 16 + row16] = o[sl][i];
         }
     }
-    if (lane < G) {
+    if (lane < gn) {
         comb_ml[wave][lane][0] = m_run;  // -inf for a wavefront without tiles
         comb_ml[wave][lane][1] = l_run;
     }
     __syncthreads();
 
     // Combine the four wavefronts in fixed order: thread -> (head, 4 dims).
-    constexpr int ITEMS = G * D / 4;
+    const int items = gn * dn / 4;
     const bool final_write = nsplit == 1;
     // Partials are stored by logical partition index, the order the merge
     // reads them in, whatever the launch order.
-    const int64_t part = ((int64_t)(tab.split_begin(b) + split) * a.kv_heads + kvh) * G;
-    for (int it = tid; it < ITEMS; it += 64 * kWaves) {
-        const int g = it / (D / 4);
-        const int d = (it % (D / 4)) * 4;
+    const int64_t part = ((int64_t)(tab.split_begin(b) + split) * a.kv_heads + kvh) * gn;
+    for (int it = tid; it < items; it += 64 * kWaves) {
+        const int g = it / (dn / 4);
+        const int d = (it % (dn / 4)) * 4;
         float m = -INFINITY;
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) m = fmaxf(m, comb_ml[w][g][0]);
@@ -467,16 +504,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void decode_kernel(DeviceArgs a) {
             uint2 packed;
             packed.x = pack_bf16x2(ov.x / l, ov.y / l);
             packed.y = pack_bf16x2(ov.z / l, ov.w / l);
-            *reinterpret_cast<uint2 *>(a.out + ((int64_t)b * a.q_heads + qh0 + g) * D + d) = packed;
+            *reinterpret_cast<uint2 *>(a.out + ((int64_t)b * a.q_heads + qh0 + g) * dn + d) = packed;
         } else if constexpr (FUSED) {
             // Agent-scope atomic stores: the merging workgroup may run on
             // another XCD.
-            float *pa = a.partial_acc + (part + g) * D + d;
+            float *pa = a.partial_acc + (part + g) * dn + d;
             store_coherent2(pa, ov.x, ov.y);
             store_coherent2(pa + 2, ov.z, ov.w);
             if (d == 0) store_coherent2(a.partial_ml + (part + g) * 2, m, l);
         } else {
-            *reinterpret_cast<float4 *>(a.partial_acc + (part + g) * D + d) = ov;
+            *reinterpret_cast<float4 *>(a.partial_acc + (part + g) * dn + d) = ov;
             if (d == 0) *reinterpret_cast<float2 *>(a.partial_ml + (part + g) * 2) = make_float2(m, l);
         }
     }
@@ -537,10 +574,11 @@ __device__ __forceinline__ void merge_splits(const DeviceArgs &a, int b, int kvh
     const int nsplit = tab.split_begin(b + 1) - tab.split_begin(b);
     const int s0 = tab.split_begin(b);
     const float c = a.scale_log2e;
-    const int qh0 = kvh * G;
-    for (int it = tid; it < G * D / 4; it += nthreads) {
-        const int g = it / (D / 4);
-        const int d = (it % (D / 4)) * 4;
+    const int gn = group_of<G>(a), dn = dim_of<D, G>(a);
+    const int qh0 = kvh * gn;
+    for (int it = tid; it < gn * dn / 4; it += nthreads) {
+        const int g = it / (dn / 4);
+        const int d = (it % (dn / 4)) * 4;
         float m = -INFINITY, l = 0.0f;
         float4 ov = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         auto fold = [&](float2 ml, float4 x) {
@@ -552,7 +590,7 @@ __device__ __forceinline__ void merge_splits(const DeviceArgs &a, int b, int kvh
             ov.z = fmaf(ov.z, wo, x.z * wn); ov.w = fmaf(ov.w, wo, x.w * wn);
             m = m_new;
         };
-        auto index = [&](int s) { return ((int64_t)(s0 + s) * a.kv_heads + kvh) * G + g; };
+        auto index = [&](int s) { return ((int64_t)(s0 + s) * a.kv_heads + kvh) * gn + g; };
         if (coherent) {
             // The merge ends the call, so all loads of a batch of K
             // partitions go out before its first fold (3K pair loads, one
@@ -565,7 +603,7 @@ __device__ __forceinline__ void merge_splits(const DeviceArgs &a, int b, int kvh
 #pragma unroll
                     for (int j = 0; j < K; ++j) {
                         const int64_t idx = index(min(sb + j, nsplit - 1));
-                        const float *pa = a.partial_acc + idx * D + d;
+                        const float *pa = a.partial_acc + idx * dn + d;
                         ml[j] = load_coherent2(a.partial_ml + idx * 2);
                         x0[j] = load_coherent2(pa);
                         x1[j] = load_coherent2(pa + 2);
@@ -583,13 +621,13 @@ __device__ __forceinline__ void merge_splits(const DeviceArgs &a, int b, int kvh
             for (int s = 0; s < nsplit; ++s) {
                 const int64_t idx = index(s);
                 fold(*reinterpret_cast<const float2 *>(a.partial_ml + idx * 2),
-                     *reinterpret_cast<const float4 *>(a.partial_acc + idx * D + d));
+                     *reinterpret_cast<const float4 *>(a.partial_acc + idx * dn + d));
             }
         }
         uint2 packed;
         packed.x = pack_bf16x2(ov.x / l, ov.y / l);
         packed.y = pack_bf16x2(ov.z / l, ov.w / l);
-        *reinterpret_cast<uint2 *>(a.out + ((int64_t)b * a.q_heads + qh0 + g) * D + d) = packed;
+        *reinterpret_cast<uint2 *>(a.out + ((int64_t)b * a.q_heads + qh0 + g) * dn + d) = packed;
     }
 }
 
@@ -602,8 +640,8 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DeviceArgs a) {
     merge_splits<D, G>(a, b, kvh, threadIdx.x, 256, false);
 }
 
-// Any-geometry fallback (head_dim not 64/128, or groups outside 1/2/4/8):
-// one wavefront per (sequence, query head), 64-token tiles, one token per
+// Any-geometry fallback (head_dim above 128, groups above 16, unaligned
+// pointers): one wavefront per (sequence, query head), 64-token tiles, one token per
 // lane for Q.K, dims across lanes for P.V.  Same addressing rule as the fast
 // kernel, so dense and paged stay bit-identical here too.
 template <bool PAGED>
@@ -903,11 +941,31 @@ struct TablePlan {
     size_t word_bytes = 0, half_bytes = 0;
 };
 
+// Geometries with a kernel variant of their own.
+bool fixed_geometry(int head_dim, int group) {
+    return (head_dim == 64 || head_dim == 128) &&
+           (group == 1 || group == 2 || group == 4 || group == 8 || group == 16);
+}
+
+// Launches the MFMA kernel takes: its fixed geometries, and through the
+// run-time variant every other head_dim up to 128 and group up to 16 whose
+// buffers are aligned for its 16-byte loads (rows are: head_dim % 8 == 0) and
+// 8-byte stores; what is left runs one wavefront per query head.  Measured
+// (8 sequences of 500 .. 4,000 tokens, 24/8 heads of 128, 73 MB of K and V): 2,969 us with one
+// wavefront per query head, 19.3 us here.
+bool decode_mfma(const DecodeLaunch &l) {
+    const int group = l.q_heads / l.kv_heads;
+    if (fixed_geometry(l.head_dim, group)) return true;
+    const uintptr_t loads = reinterpret_cast<uintptr_t>(l.q) | reinterpret_cast<uintptr_t>(l.k) |
+                            reinterpret_cast<uintptr_t>(l.v);
+    return l.head_dim <= 128 && group <= 16 && (loads & 15) == 0 && (reinterpret_cast<uintptr_t>(l.out) & 7) == 0;
+}
+
 TablePlan table_plan(const DecodeLaunch &l) {
     TablePlan p;
     for (int i = 0; i < l.batch; ++i) p.total += decode_splits(l.seq_len[i], l.split_tokens);
     const int64_t items = (int64_t)p.total * l.kv_heads;
-    p.lists = decode_fast_path(l.head_dim, l.q_heads / l.kv_heads) && !l.separate_merge && items > kListBins &&
+    p.lists = decode_mfma(l) && !l.separate_merge && items > kListBins &&
               items <= kMaxListItems;
     const int64_t halves = l.batch + (p.lists ? kListBins + 1 + items : 0);
     p.inline_args = l.batch <= kInlineBatch && halves <= kInlineHalves;
@@ -921,10 +979,6 @@ size_t decode_table_bytes(const DecodeLaunch &l) {
     return p.inline_args ? 0 : p.word_bytes + p.half_bytes;
 }
 
-bool decode_fast_path(int head_dim, int group) {
-    return (head_dim == 64 || head_dim == 128) &&
-           (group == 1 || group == 2 || group == 4 || group == 8 || group == 16);
-}
 
 namespace {
 
@@ -932,7 +986,7 @@ hipError_t launch_kernels(const DeviceArgs &a, const DecodeLaunch &l, int total,
                           hipStream_t stream) {
     const int group = l.q_heads / l.kv_heads;
     const bool nt = kv_tokens * l.kv_heads * l.head_dim * 2 * 2 >= kNonTemporalBytes;
-    if (!decode_fast_path(l.head_dim, group)) {
+    if (!decode_mfma(l)) {
         const dim3 grid((unsigned)(l.batch * l.q_heads));
         if (l.paged)
             hipLaunchKernelGGL((decode_generic_kernel<true>), grid, dim3(64), 0, stream, a, l.head_dim);
@@ -954,7 +1008,8 @@ hipError_t launch_kernels(const DeviceArgs &a, const DecodeLaunch &l, int total,
     MSLIM_DECODE_CASE(64, 2)
     MSLIM_DECODE_CASE(64, 1)
 #undef MSLIM_DECODE_CASE
-    return hipErrorInvalidValue;
+    if (l.head_dim <= 64) return launch_fast<64, 0>(a, l.paged, nt, total, merge, !l.separate_merge, stream);
+    return launch_fast<128, 0>(a, l.paged, nt, total, merge, !l.separate_merge, stream);
 }
 
 }  // namespace
@@ -971,7 +1026,7 @@ hipError_t launch_decode(const DecodeLaunch &l, hipStream_t stream) {
     if (l.paged) {
         while ((1 << a.page_shift) < l.page_tokens) ++a.page_shift;
     }
-    a.batch = l.batch; a.q_heads = l.q_heads; a.kv_heads = l.kv_heads;
+    a.batch = l.batch; a.q_heads = l.q_heads; a.kv_heads = l.kv_heads; a.head_dim = l.head_dim;
     a.split_tokens = l.split_tokens;
     a.scale_log2e = l.scale * kLog2e;
     const TablePlan plan = table_plan(l);

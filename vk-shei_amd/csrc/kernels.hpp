@@ -63,11 +63,10 @@ inline int decode_splits(int tokens, int split_tokens) {
 // equal lengths, smaller for ragged lengths when that evens out the busiest
 // CU's load; a multiple of 256 in 256..16384, or 128 for tiny batches.
 int decode_auto_split_tokens(const int32_t *seq_lens, int batch, int kv_heads);
-// True when the MFMA fast path covers this geometry.
-bool decode_fast_path(int head_dim, int group);
 hipError_t launch_decode(const DecodeLaunch &a, hipStream_t stream);
 // Bytes of the device copy of a launch's tables (0: they fit the kernel
-// arguments).  Needs seq_len, split_tokens, the geometry and separate_merge.
+// arguments).  Needs seq_len, split_tokens, the geometry, the buffers and
+// separate_merge.
 size_t decode_table_bytes(const DecodeLaunch &l);
 // Split-partial bytes a decode launch of this shape needs.
 size_t decode_partial_bytes(const DecodeLaunch &l);
