@@ -70,3 +70,50 @@ def test_decode_any_group(ctx, qh, kvh, d):
         for i in range(b):
             _check(from_torch(dense[i]), ref[i], vb[i], f"split {split} sequence {i}")
             _check(from_torch(plain[i]), ref[i], vb[i], f"unaligned, split {split} sequence {i}")
+
+
+# (queries, prior): one row, tile and row-block edges, a remainder after a
+# prior, and lengths whose launches split their row blocks.
+PREFILL = [(1, 0), (33, 0), (257, 130), (600, 1500)]
+
+
+@pytest.mark.parametrize("queries,prior", PREFILL)
+@pytest.mark.parametrize("qh,kvh,d", [(3, 1, 128), (10, 2, 64), (6, 1, 128), (18, 3, 64), (14, 2, 128)])
+def test_prefill_any_group(ctx, qh, kvh, d, queries, prior):
+    rng = np.random.default_rng(queries * 100 + qh)
+    t = queries + prior
+    qb, kb, vb = (normal_bf16(rng, s) for s in ((queries, qh, d), (t, kvh, d), (t, kvh, d)))
+    _check_prefill(ctx, rng, qb, kb, vb, queries, prior, qh, kvh, d)
+
+
+@pytest.mark.parametrize("qh,kvh,d", [(3, 1, 128), (6, 1, 64)])
+def test_prefill_any_group_moving_reference(ctx, qh, kvh, d):
+    # scores that climb past the lazy bound tile after tile, then one so far
+    # above the reference that its first p overflows
+    rng = np.random.default_rng(d)
+    queries = 400
+    k = 0.4 * (128.0 / d) ** 0.5 * np.arange(queries, dtype=np.float32) / 64.0
+    k[330] = 20.0 * (128.0 / d) ** 0.5
+    qb = oracle.write_bf16(np.ones((queries, qh, d), np.float32)).reshape(queries, qh, d)
+    kb = oracle.write_bf16(np.broadcast_to(k[:, None, None], (queries, kvh, d))).reshape(queries, kvh, d)
+    _check_prefill(ctx, rng, qb, kb, normal_bf16(rng, (queries, kvh, d)), queries, 0, qh, kvh, d)
+
+
+def _check_prefill(ctx, rng, qb, kb, vb, queries, prior, qh, kvh, d):
+    q, k, v = to_torch(qb), to_torch(kb), to_torch(vb)
+    whole, unsplit, plain = (torch.empty_like(q) for _ in range(3))
+    ctx.prefill_causal(q, k, v, whole, queries, prior, qh, kvh, d)
+    try:
+        ctx.set_prefill_split(False)
+        ctx.prefill_causal(q, k, v, unsplit, queries, prior, qh, kvh, d)
+    finally:
+        ctx.set_prefill_split(True)
+    ctx.prefill_causal(_unaligned(q), k, v, plain, queries, prior, qh, kvh, d)  # the any-geometry kernel
+    torch.cuda.synchronize()
+    rows = sorted({0, queries // 2, queries - 1} | {int(r) for r in rng.integers(0, queries, 12)})
+    outs = [from_torch(x) for x in (whole, unsplit, plain)]
+    for r in rows:
+        n = prior + r + 1
+        ref = oracle.cpu_reference_decode(oracle.read_bf16(qb[r]), kb[:n], vb[:n], 1, qh, kvh, d)[1]
+        for name, got in zip(("split", "unsplit", "unaligned"), outs):
+            _check(got[r], ref, vb[:n], f"{name} row {r}")

@@ -91,7 +91,8 @@ struct PrefillLaunch {
     bool pool_allowed;   // hand the shortest row blocks out at run time (unsplit launches)
     int *pool_counter;   // one int, zero between launches, when prefill_pool_items() > 0
 };
-bool prefill_fast_path(int head_dim, int group);
+// True when the MFMA kernel covers this launch (geometry and alignment).
+bool prefill_mfma(const PrefillLaunch &l);
 // Row blocks per XCD that an unsplit launch hands out at run time (0: none).
 int prefill_pool_items(const PrefillLaunch &l);
 // How a launch splits its row blocks: chunk_tiles == 0 means no split.

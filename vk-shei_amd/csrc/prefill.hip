@@ -126,7 +126,14 @@ struct Swz {
 // are issued by inline assembly and waited for explicitly ahead of a
 // fence-free barrier.  HW heads x (8/HW) row blocks of 32 rows per
 // workgroup.
-template <int D, int HW>
+//
+// WIDE serves the groups that have no 2, 4 or 8 heads to share a tile evenly
+// (3, 5, 6, 7, ...): Q enters the MFMAs as it is and the scale is applied to
+// the f32 score (one FMA per score in place of the seed), and P is kept to 16
+// bits of mantissa as two BF16 parts, each with its own P.V MFMA.  Those
+// groups have had f32 scores and probabilities in the any-geometry kernel,
+// whose error against 64 bits this matches.
+template <int D, int HW, bool WIDE>
 __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
     constexpr int ST = 4;  // LDS stages
     constexpr int WAVES = 8;
@@ -219,10 +226,12 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
         const uint16_t *qp = a.q + ((int64_t)qrow * a.q_heads + head) * D + half * 8;
 #pragma unroll
         for (int j = 0; j < KS; ++j) qf[j] = *reinterpret_cast<const bf16x8_t *>(qp + j * 16);
+        if constexpr (!WIDE) {
 #pragma unroll
-        for (int j = 0; j < KS; ++j)
+            for (int j = 0; j < KS; ++j)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) qf[j][e] = (__bf16)((float)qf[j][e] * c);
+                for (int e = 0; e < 8; ++e) qf[j][e] = (__bf16)((float)qf[j][e] * c);
+        }
     }
     // Q has landed before any K/V copy is issued (no wait inside the loop
     // may hold back copies in flight).
@@ -304,6 +313,7 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
     bool rescale_pending = false;
     floatx16_t s[2];
     bf16x8_t pprev[2][2];  // P of the previous tile, [key block][16-key half]
+    bf16x8_t plow[2][2];   // WIDE: its low parts
 
     const int q4 = lane >> 4;
     const int rr = (lane & 15) >> 2;
@@ -333,7 +343,7 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
     // S^T of one tile from K stage kst; seeded: relative to the reference
     // (first tile of the workgroup: absolute, the reference is not known yet).
     auto qk = [&](int kst, auto seeded_tag, auto &&mid) __attribute__((always_inline)) {
-        constexpr bool seeded = decltype(seeded_tag)::value;
+        constexpr bool seeded = decltype(seeded_tag)::value && !WIDE;
         auto kfrag = [&](int ks, int kb) __attribute__((always_inline)) {
             return lds_read_b128(kaddr[ks] + kst * STAGE + kb * 32 * D * 2);
         };
@@ -379,12 +389,24 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
     // and the next): exp2 of the score less `sub` (none for scores already
     // relative to the reference), BF16 pack, and the row sum of the packed P
     // that feeds the MFMA.
-    auto score_pair = [&](int pidx, uint32_t (&pw)[2][8], float &psum, auto sub_tag, float sub)
+    // WIDE: the score times c less `sub`, and the pair's low parts beside it.
+    auto score_pair = [&](int pidx, uint32_t (&pw)[2][8], uint32_t (&pl)[2][8], float &psum, auto sub_tag, float sub)
         __attribute__((always_inline)) {
         constexpr bool do_sub = decltype(sub_tag)::value;
         const int kb = pidx / 8, r = (pidx % 8) * 2;
         bf16x2_t pp;
-        if constexpr (do_sub) {
+        if constexpr (WIDE) {
+            const float p0 = __builtin_amdgcn_exp2f(fmaf(s[kb][r], c, -sub));
+            const float p1 = __builtin_amdgcn_exp2f(fmaf(s[kb][r + 1], c, -sub));
+            pp[0] = (__bf16)p0;
+            pp[1] = (__bf16)p1;
+            bf16x2_t low;
+            low[0] = (__bf16)(p0 - (float)pp[0]);
+            low[1] = (__bf16)(p1 - (float)pp[1]);
+            pl[kb][r >> 1] = __builtin_bit_cast(uint32_t, low);
+            psum = add_bf16_pair(low, psum);
+            pin_value(pl[kb][r >> 1]);
+        } else if constexpr (do_sub) {
             pp[0] = (__bf16)__builtin_amdgcn_exp2f(s[kb][r] - sub);
             pp[1] = (__bf16)__builtin_amdgcn_exp2f(s[kb][r + 1] - sub);
         } else {
@@ -419,6 +441,7 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
             const int mt = n % MT, t = (n / MT) % 2, kb = n / (2 * MT);
             __builtin_amdgcn_sched_barrier(0);
             o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vhead[n], pprev[kb][t], o[mt], 0, 0, 0);
+            if constexpr (WIDE) o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vhead[n], plow[kb][t], o[mt], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -439,7 +462,7 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
             vq[1] = vfrag(vst, N0 + 1);
         }
         float mx = 0.0f, psum = 0.0f;
-        uint32_t pw[2][8];
+        uint32_t pw[2][8], pl[2][8];
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
             const int n = N0 + i;
@@ -450,6 +473,8 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
             if constexpr (do_pv) {
                 const int mt = n % MT, t = (n / MT) % 2, kb = n / (2 * MT);
                 o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vq[i % 3], pprev[kb][t], o[mt], 0, 0, 0);
+                if constexpr (WIDE)
+                    o[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vq[i % 3], plow[kb][t], o[mt], 0, 0, 0);
             }
             if constexpr (do_sm && first) {
                 // The workgroup's first tile: the reference is still -inf, so
@@ -464,10 +489,11 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
 #pragma unroll
                     for (int r = 1; r < 15; r += 2) mx = __builtin_fmaxf(__builtin_fmaxf(mx, s[1][r]), s[1][r + 1]);
                     m_used = half_pair_max(__builtin_fmaxf(mx, s[1][15]));
+                    if constexpr (WIDE) m_used *= c;
                 } else {
 #pragma unroll
                     for (int pidx = 0; pidx < 16; ++pidx)
-                        if (2 + (pidx * (NL - 2)) / 16 == i) score_pair(pidx, pw, psum, Yes{}, m_used);
+                        if (2 + (pidx * (NL - 2)) / 16 == i) score_pair(pidx, pw, pl, psum, Yes{}, m_used);
                     pin_value(psum);
                 }
             } else if constexpr (do_sm) {
@@ -476,7 +502,7 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
                 // test in the last slot.
 #pragma unroll
                 for (int pidx = 0; pidx < 16; ++pidx)
-                    if ((pidx * (NL - 1)) / 16 == i) score_pair(pidx, pw, psum, No{}, 0.0f);
+                    if ((pidx * (NL - 1)) / 16 == i) score_pair(pidx, pw, pl, psum, No{}, WIDE ? m_used : 0.0f);
                 pin_value(psum);
                 // Every p of the tile is at most its row sum, so the reference
                 // need not move while each row sum stays within 2^8 (exact: the
@@ -484,7 +510,8 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
                 // the first tile; also when a p overflowed) take the tile's row
                 // maximum, move the reference for the rows that exceed it, and
                 // recompute the tile's P under the new one.
-                if (i == NL - 1 && wave_any(psum > kLazyBound)) {
+                // (WIDE: the low part of a p that overflowed is NaN.)
+                if (i == NL - 1 && wave_any(WIDE ? !(psum <= kLazyBound) : psum > kLazyBound)) {
                     mx = s[0][0];
 #pragma unroll
                     for (int r = 1; r < 15; r += 2) mx = __builtin_fmaxf(__builtin_fmaxf(mx, s[0][r]), s[0][r + 1]);
@@ -493,7 +520,7 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
                     for (int r = 1; r < 15; r += 2) mx = __builtin_fmaxf(__builtin_fmaxf(mx, s[1][r]), s[1][r + 1]);
                     mx = half_pair_max(__builtin_fmaxf(mx, s[1][15]));
                     // The row's maximum above the reference (0: it stays).
-                    const float shift = fmaxf(mx, 0.0f);
+                    const float shift = fmaxf(WIDE ? fmaf(mx, c, -m_used) : mx, 0.0f);
                     const float alpha = __builtin_amdgcn_exp2f(-shift);
                     l_run *= alpha;
                     alpha_pending = alpha;
@@ -503,7 +530,7 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
                     for (int r = 0; r < 16; ++r) seed[r] = -m_used;
                     psum = 0.0f;
 #pragma unroll
-                    for (int pidx = 0; pidx < 16; ++pidx) score_pair(pidx, pw, psum, Yes{}, shift);
+                    for (int pidx = 0; pidx < 16; ++pidx) score_pair(pidx, pw, pl, psum, Yes{}, WIDE ? m_used : shift);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -516,6 +543,10 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
                 for (int t = 0; t < 2; ++t) {
                     const uint4 u = {pw[kb][4 * t], pw[kb][4 * t + 1], pw[kb][4 * t + 2], pw[kb][4 * t + 3]};
                     pprev[kb][t] = __builtin_bit_cast(bf16x8_t, u);
+                    if constexpr (WIDE) {
+                        const uint4 w = {pl[kb][4 * t], pl[kb][4 * t + 1], pl[kb][4 * t + 2], pl[kb][4 * t + 3]};
+                        plow[kb][t] = __builtin_bit_cast(bf16x8_t, w);
+                    }
                 }
         }
     };
@@ -767,7 +798,7 @@ __global__ __launch_bounds__(64) void prefill_generic_kernel(PrefillArgs a, int 
     }
 }
 
-template <int D, int HW>
+template <int D, int HW, bool WIDE = false>
 hipError_t launch_mfma(const PrefillArgs &a, hipStream_t stream) {
     constexpr int RW = 32 * (8 / HW);
     const int group = a.q_heads / a.kv_heads;
@@ -775,12 +806,16 @@ hipError_t launch_mfma(const PrefillArgs &a, hipStream_t stream) {
     const int per_xcd = (total + kXcds - 1) / kXcds;
     const int spare = a.pool_items ? kPoolSpare : 0;
     const unsigned grid = a.chunk_tiles ? (unsigned)a.items : (unsigned)((per_xcd + spare) * kXcds);
-    hipLaunchKernelGGL((prefill_mfma_kernel<D, HW>), dim3(grid), dim3(512), 0, stream, a);
+    hipLaunchKernelGGL((prefill_mfma_kernel<D, HW, WIDE>), dim3(grid), dim3(512), 0, stream, a);
     return hipGetLastError();
 }
 
 // Heads per workgroup: the largest of 8, 4, 2, 1 that divides the group.
-int heads_per_workgroup(int group) { return group % 8 == 0 ? 8 : group % 4 == 0 ? 4 : group; }
+int heads_per_workgroup(int group) { return group % 8 == 0 ? 8 : group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1; }
+
+// Groups whose heads the kernel with the pre-scaled Q shares out; the others
+// take its WIDE form.
+bool even_group(int group) { return group == 1 || group == 2 || group % 4 == 0; }
 
 // Key tiles of row block rb.
 int row_block_tiles(const PrefillLaunch &l, int rows_per_block, int rb) {
@@ -790,8 +825,17 @@ int row_block_tiles(const PrefillLaunch &l, int rows_per_block, int rb) {
 
 }  // namespace
 
-bool prefill_fast_path(int head_dim, int group) {
-    return (head_dim == 64 || head_dim == 128) && (group == 1 || group == 2 || group % 4 == 0);
+// Launches the MFMA kernel takes: head_dim 64 or 128, for the groups of its
+// WIDE form with buffers aligned for the 16-byte loads and 8-byte stores; what
+// is left runs one wavefront per query row and head.  Measured (1,001 queries
+// of 24/8 heads of 128): 5,523 us with a wavefront per row and head, 30.1 us
+// here.
+bool prefill_mfma(const PrefillLaunch &l) {
+    if (l.head_dim != 64 && l.head_dim != 128) return false;
+    if (even_group(l.q_heads / l.kv_heads)) return true;
+    const uintptr_t loads = reinterpret_cast<uintptr_t>(l.q) | reinterpret_cast<uintptr_t>(l.k) |
+                            reinterpret_cast<uintptr_t>(l.v);
+    return (loads & 15) == 0 && (reinterpret_cast<uintptr_t>(l.out) & 7) == 0;
 }
 
 namespace {
@@ -860,8 +904,7 @@ PrefillSplit plan_split(const PrefillLaunch &l);
 // host time, so plans are kept per shape (a decoder repeats a few prompt-chunk
 // shapes over every layer and sequence).
 PrefillSplit prefill_split_plan(const PrefillLaunch &l) {
-    const int group = l.q_heads / l.kv_heads;
-    if (!l.split_allowed || !prefill_fast_path(l.head_dim, group)) return PrefillSplit{};
+    if (!l.split_allowed || !prefill_mfma(l)) return PrefillSplit{};
     const std::array<int, 5> key = {l.queries, l.prior, l.q_heads, l.kv_heads, l.head_dim};
     static std::mutex lock;
     static std::map<std::array<int, 5>, PrefillSplit> plans;
@@ -938,7 +981,7 @@ PrefillSplit plan_split(const PrefillLaunch &l) {
 
 int prefill_pool_items(const PrefillLaunch &l) {
     const int group = l.q_heads / l.kv_heads;
-    if (!l.pool_allowed || !prefill_fast_path(l.head_dim, group) || prefill_split_plan(l).chunk_tiles) return 0;
+    if (!l.pool_allowed || !prefill_mfma(l) || prefill_split_plan(l).chunk_tiles) return 0;
     const int hw = heads_per_workgroup(group);
     const int rows = 32 * (8 / hw);
     const int64_t total = (int64_t)((l.queries + rows - 1) / rows) * l.kv_heads * (group / hw);
@@ -960,7 +1003,7 @@ hipError_t launch_prefill(const PrefillLaunch &l, hipStream_t stream) {
     a.q_heads = l.q_heads; a.kv_heads = l.kv_heads;
     a.scale_log2e = l.scale * kLog2e;
     const int group = l.q_heads / l.kv_heads;
-    if (!prefill_fast_path(l.head_dim, group)) {
+    if (!prefill_mfma(l)) {
         hipLaunchKernelGGL(prefill_generic_kernel, dim3((unsigned)(l.queries * l.q_heads)), dim3(64), 0,
                            stream, a, l.head_dim);
         return hipGetLastError();
@@ -1022,6 +1065,10 @@ hipError_t launch_prefill(const PrefillLaunch &l, hipStream_t stream) {
         if (!l.pool_counter) return hipErrorInvalidValue;
         a.pool_items = pool;
         a.pool_counter = l.pool_counter;
+    }
+    if (!even_group(group)) {
+        if (l.head_dim == 128) return hw == 2 ? launch_mfma<128, 2, true>(a, stream) : launch_mfma<128, 1, true>(a, stream);
+        return hw == 2 ? launch_mfma<64, 2, true>(a, stream) : launch_mfma<64, 1, true>(a, stream);
     }
     if (l.head_dim == 128) {
         if (hw == 8) return launch_mfma<128, 8>(a, stream);
