@@ -331,6 +331,13 @@ void *mslim_attn_ctx_new(void) {
         delete c;
         return nullptr;
     }
+    // Partials of split projections, enough for every shape of inner < 8192:
+    // those calls allocate nothing, so their first one may be under capture.
+    if (check_hip(hipMalloc(&c->proj_partial, mslim::kProjPartialBytes), "hipMalloc projection partials")) {
+        delete c;
+        return nullptr;
+    }
+    c->proj_partial_bytes = mslim::kProjPartialBytes;
     // The allocation-free decode's fixed partials array: its address on this
     // device is taken here, once, so that entry point's first call loads
     // nothing.
@@ -1268,15 +1275,15 @@ int mslim_attn_record_payloads(void *ctx, void *k_pool, void *v_pool, int64_t po
     return check_hip(mslim::launch_record_payloads(l, direction == 0, c.stream), "record payload launch");
 }
 
-// The fp32 partials of a split projection (none for other shapes), in a
-// context buffer that only grows (stage code 400 if it cannot).
-// `outputs`: products x the matrices' total rows (2 x rows for SwiGLU).
-static int proj_partials(Context &c, int inner, int64_t outputs, int tokens, float **partial) {
+// The fp32 partials of a launch's split products (none when nothing is split),
+// in a context buffer that only grows (stage code 400 if it cannot).
+// `products`: sums per output, 2 for SwiGLU.
+static int proj_partials(Context &c, std::initializer_list<int> rows, int products, int inner, int tokens,
+                         float **partial) {
     *partial = nullptr;
-    const int split = mslim::proj_ksplit(inner);
-    if (split < 2) return 0;
-    if (grow_device(c, &c.proj_partial, &c.proj_partial_bytes, (size_t)split * outputs * tokens * sizeof(float),
-                    "hipMalloc projection partials"))
+    const size_t floats = mslim::proj_partial_floats(rows.begin(), (int)rows.size(), products, inner, tokens);
+    if (!floats) return 0;
+    if (grow_device(c, &c.proj_partial, &c.proj_partial_bytes, floats * sizeof(float), "hipMalloc projection partials"))
         return 400;
     *partial = static_cast<float *>(c.proj_partial);
     return 0;
@@ -1294,7 +1301,7 @@ static int project(Context &c, const void *weight, const void *input, void *outp
                    ? 404
                    : 0;
     float *partial = nullptr;
-    if (int rc = proj_partials(c, inner, rows, tokens, &partial)) return rc;
+    if (int rc = proj_partials(c, {rows}, 1, inner, tokens, &partial)) return rc;
     return check_hip(mslim::launch_proj(&m, 1, x, inner, tokens, partial, c.stream), "projection launch") ? 404 : 0;
 }
 
@@ -1356,7 +1363,7 @@ int mslim_attn_gemm_bf16_add(void *ctx, const void *weight, const void *input, c
     }
     const mslim::SkinnyMatrix m{w, static_cast<uint16_t *>(output), rows};
     float *partial = nullptr;
-    if (int rc = proj_partials(c, inner, rows, tokens, &partial)) return rc;
+    if (int rc = proj_partials(c, {rows}, 1, inner, tokens, &partial)) return rc;
     return check_hip(mslim::launch_proj_add(m, static_cast<const uint16_t *>(residual), x, inner, tokens, partial,
                                             c.stream),
                      "projection launch")
@@ -1384,7 +1391,7 @@ int mslim_attn_gemm_swiglu(void *ctx, const void *gate_weight, const void *up_we
                    : 0;
     }
     float *partial = nullptr;
-    if (int rc = proj_partials(c, inner, 2 * (int64_t)rows, tokens, &partial)) return rc;
+    if (int rc = proj_partials(c, {rows}, 2, inner, tokens, &partial)) return rc;
     return check_hip(mslim::launch_proj_swiglu(static_cast<const uint16_t *>(gate_weight),
                                                static_cast<const uint16_t *>(up_weight),
                                                static_cast<uint16_t *>(output), rows, x, inner, tokens,
@@ -1421,7 +1428,7 @@ int mslim_attn_gemm_qkv(void *ctx, const void *q_weight, const void *k_weight, c
         {static_cast<const uint16_t *>(k_weight), static_cast<uint16_t *>(k_out), kv_rows},
         {static_cast<const uint16_t *>(v_weight), static_cast<uint16_t *>(v_out), kv_rows}};
     float *partial = nullptr;
-    if (int rc = proj_partials(c, inner, (int64_t)q_rows + 2 * (int64_t)kv_rows, tokens, &partial)) return rc;
+    if (int rc = proj_partials(c, {q_rows, kv_rows, kv_rows}, 1, inner, tokens, &partial)) return rc;
     return check_hip(mslim::launch_proj(m, 3, static_cast<const uint16_t *>(input), inner, tokens, partial, c.stream),
                      "projection launch")
                ? 404
@@ -1495,7 +1502,7 @@ static int rmsnorm_gemm_qkv_locked(Context &c, const void *norm_weight, float ep
                    ? 404
                    : 0;
     float *partial = nullptr;
-    if (int rc = proj_partials(c, inner, (int64_t)q_rows + 2 * (int64_t)kv_rows, tokens, &partial)) return rc;
+    if (int rc = proj_partials(c, {q_rows, kv_rows, kv_rows}, 1, inner, tokens, &partial)) return rc;
     return check_hip(mslim::launch_proj(m, 3, static_cast<const uint16_t *>(x), inner, tokens, partial, c.stream),
                      "projection launch")
                ? 404
@@ -1548,7 +1555,7 @@ int mslim_attn_rmsnorm_gemm_swiglu(void *ctx, const void *norm_weight, float eps
                    ? 404
                    : 0;
     float *partial = nullptr;
-    if (int rc = proj_partials(c, inner, 2 * (int64_t)rows, tokens, &partial)) return rc;
+    if (int rc = proj_partials(c, {rows}, 2, inner, tokens, &partial)) return rc;
     return check_hip(mslim::launch_proj_swiglu(gw, uw, static_cast<uint16_t *>(output), rows,
                                                static_cast<const uint16_t *>(x), inner, tokens, c.swiglu_table,
                                                partial, c.stream),

@@ -294,10 +294,12 @@ hipError_t launch_skinny_swiglu(const uint16_t *w_gate, const uint16_t *w_up, ui
 // The same products for any number of token rows (csrc/proj.hip): the tiled
 // MFMA kernel when inner is a multiple of 64 and x and the weights are
 // 16-byte aligned, one wavefront per output otherwise.  Same epilogues.
-// Split launches (proj_ksplit(inner) > 1) keep fp32 partials in `partial`:
-// proj_ksplit * products * tokens * (sum of the matrices' rows) floats, with
-// products 2 for SwiGLU (gate and up) and 1 otherwise.
-int proj_ksplit(int inner);
+// Split launches keep fp32 partials in `partial`: proj_partial_floats floats
+// (0: not split), with products 2 for SwiGLU (gate and up) and 1 otherwise.
+size_t proj_partial_floats(const int *rows, int count, int products, int inner, int tokens);
+// Partials that every launch of inner < 8192 fits in: a context holds as much
+// from the start, so those launches never allocate.
+constexpr size_t kProjPartialBytes = (size_t)48 << 20;
 hipError_t launch_proj(const SkinnyMatrix *m, int count, const uint16_t *x, int inner, int tokens, float *partial,
                        hipStream_t stream);
 hipError_t launch_proj_add(const SkinnyMatrix &m, const uint16_t *resid, const uint16_t *x, int inner, int tokens,

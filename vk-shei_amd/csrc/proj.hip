@@ -5,18 +5,21 @@
 // gpu_llm.cl:553-683, :1253-1383, driven from gpu_llm/prefill.rs:132-290;
 // tv_hip_matrix_multiply, hipblaslt_bridge.cpp:203-233, under its HIP
 // backend) as one hand-written gfx950 kernel:
-//   * a workgroup of four wavefronts (one per SIMD) owns 128 weight rows x BN
-//     token rows of the output; each wavefront WM x 64 (WM = 32, BN = 64 for
-//     launches of few tiles; WM = 64, BN = 128 otherwise), as blocks of
+//   * a workgroup owns a tile of 64 or 128 weight rows x 64 to 256 token rows of
+//     the output, its wavefronts 32 x 32 to 64 x 64 of it, as blocks of
 //     v_mfma_f32_32x32x16_bf16 with the weights as A (rows = M) and the token
 //     rows as B (N), so a lane ends up with 4 consecutive output rows of one
 //     token per 4 accumulators;
 //   * both operands are K-contiguous; 64-element k-steps of both move HBM ->
-//     LDS with global_load_lds_dwordx4 into a three-stage ring (128-byte rows,
-//     16-byte slots XOR-swizzled by (row / 2) % 8, so every 16 rows of a
-//     fragment read fall in distinct banks), one barrier per k-step;
-//   * the last sub-step's MFMAs of a k-step run after the next barrier, behind
-//     the next stage's first fragment reads;
+//     LDS with global_load_lds_dwordx4 into a ring of three or four stages
+//     (128-byte rows, 16-byte slots XOR-swizzled by (row / 2) % 8, so every 16
+//     rows of a fragment read fall in distinct banks), one barrier per k-step;
+//   * fragment reads and copies are pinned between the MFMAs, and the last
+//     sub-step's MFMAs of a k-step run after the next barrier, behind the next
+//     stage's first fragment reads;
+//   * a product whose tiles would leave CUs idle is cut along k: each split
+//     writes fp32 partial sums and a second launch adds them in split order.
+//     The number of splits is a function of the product's shape alone;
 //   * tiles are dealt to XCDs in contiguous slices with the token tiles of a
 //     weight slice adjacent, so each weight row is read from HBM by one XCD;
 //   * epilogues: plain, residual add (out = BF16(resid + BF16(acc)), llm_add
@@ -24,8 +27,17 @@
 //     same tile (llm_swiglu after both), and up to three matrices with their
 //     own outputs in one launch (Q, K, V), each equal bit for bit to the
 //     plain product followed by the elementwise kernel.
-// Every output is summed by one wavefront in fixed k order, so results do not
+// Every split is summed by one wavefront in fixed k order, so results do not
 // depend on the tiling or on timing: a fused launch equals the separate ones.
+// What bounds it: up to about 100 token rows the weights' HBM stream, above
+// them the latency of first reads (about 1.5 us against a ring of 64 to 96
+// KiB; the pure MFMA loop takes two thirds of the time at 512 tokens).
+// Against 128 x 128 / 128 x 64 tiles of four wavefronts split by inner alone
+// (us, 4,096 hidden, 14,336 intermediate; O, Q-K-V, gate and up, down):
+//   20 tokens   30 / 30 / 56 / 58   ->  12 / 16 / 43 / 26
+//   128 tokens  33 / 32 / 60 / 76   ->  17 / 22 / 52 / 38
+//   300 tokens  33 / 32 / 123 / 65  ->  25 / 33 / 109 / 58
+//   512 tokens  34 / 39 / 131 / 80  ->  30 / 39 / 116 / 68
 // Shapes outside the fast path (inner not a multiple of 64, unaligned
 // pointers) run proj_generic_kernel: one wavefront per output, lane-strided
 // partial sums and a fixed reduction tree.
@@ -33,15 +45,13 @@
 #include "kernels.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace mslim {
 
 namespace {
 
-constexpr int kBM = 128;   // weight rows per workgroup tile
-constexpr int kBK = 64;    // inputs per k-step
-constexpr int kStages = 3; // LDS ring stages
-constexpr int kKAlign = kBK;  // inner must be a multiple of this for the tiled kernel
+constexpr int kKAlign = 64;   // inner must be a multiple of this for the tiled kernel
 constexpr int kXcds = 8;
 constexpr int kMaxSeg = 3;
 
@@ -51,7 +61,6 @@ struct ProjArgs {
     const uint16_t *w[kMaxSeg];
     uint16_t *out[kMaxSeg];
     int rows[kMaxSeg];
-    int first_tile[kMaxSeg + 1];  // row tiles before segment s; [segments] = all
     int segments;
     const uint16_t *w_up;   // SwiGLU: up weights beside w[0] (gate)
     const uint16_t *act_table;  // SwiGLU: swiglu_act_bf16 of every gate value
@@ -59,56 +68,73 @@ struct ProjArgs {
     const uint16_t *x;      // [tokens][inner]
     int inner, tokens;
     int n_tiles;            // token tiles
-    // ksplit > 1: workgroup (tile, s) sums k-steps [s nk / ksplit,
-    // (s + 1) nk / ksplit) into partial[s][product][out], fp32, where out
-    // runs over every segment's [tokens][rows] in segment order (out_base)
-    // and product is the gate (0) or up (1) sum of SwiGLU; a second launch
-    // adds the partials in split order and applies the epilogue.
-    int ksplit;
+    // Work items (row tile, token tile, k split) before segment s;
+    // [segments] = all.
+    int first_item[kMaxSeg + 1];
+    // ksplit[s] > 1: item (tile, k split i) sums k-steps [i nk / ksplit,
+    // (i + 1) nk / ksplit) of segment s into partial + part_base[s], fp32
+    // [ksplit][product][tokens][rows], product the gate (0) or up (1) sum of
+    // SwiGLU; a second launch adds the partials in split order and applies
+    // the epilogue.
+    int ksplit[kMaxSeg];
+    int64_t part_base[kMaxSeg];
     float *partial;
-    int64_t out_base[kMaxSeg + 1];  // [segments] = all outputs
 };
 
-// Swizzle of a row of NSL 16-byte slots: the slot XOR this.  64 banks of 4
-// bytes hold two 128-byte rows, so the 16 rows one LDS cycle serves are
-// conflict-free when the 8 rows of each parity take 8 distinct slots; a
-// 256-byte row fills the banks alone and needs 16 distinct slots.
+// Swizzle of a row of NSL 16-byte slots: the slot XOR this.  The 64 banks of
+// 4 bytes hold 16 slots, 16 / NSL rows; one LDS cycle of a fragment read
+// serves 16 rows at one slot, and they fall in distinct banks when the rows
+// that share a place modulo 16 / NSL take distinct slots.
 template <int NSL>
 __device__ __forceinline__ int proj_swz(int row) {
-    return NSL == 8 ? (row >> 1) & 7 : row & (NSL - 1);
+    return (row / (16 / NSL)) & (NSL - 1);
 }
+
+// A configuration: BM weight rows x BN token rows per workgroup, MI x NJ
+// 32 x 32 MFMA blocks per wavefront, k-steps of BK inputs in a ring of ST LDS
+// stages.
+template <int BM_, int BN_, int MI_, int NJ_, int BK_, int ST_, int WAVES_ = 4>
+struct Config {
+    static constexpr int BM = BM_, BN = BN_, MI = MI_, NJ = NJ_, BK = BK_, ST = ST_, WAVES = WAVES_;
+};
 
 // LDS of a configuration: ST stages of the weight tile(s) and the token tile;
-// the SwiGLU epilogue reuses it for the 128 KiB activation table.
+// the SwiGLU epilogue of the tiles with many outputs reuses it for the 128 KiB
+// activation table (the others read the table from L2).
 constexpr int kTableBytes = kSwigluTableEntries * 2;
-constexpr int proj_lds_bytes(int wm, int bk, int st, int epi) {
-    const int stages = st * ((epi == kSwiglu ? 2 : 1) * kBM + 64 * (4 / (kBM / wm))) * bk * 2;
-    return epi == kSwiglu && stages < kTableBytes ? kTableBytes : stages;
+template <class C>
+constexpr bool table_in_lds(int epi) {
+    return epi == kSwiglu && C::BM * C::BN >= 128 * 64;
+}
+template <class C>
+constexpr int proj_lds_bytes(int epi) {
+    const int stages = C::ST * ((epi == kSwiglu ? 2 : 1) * C::BM + C::BN) * C::BK * 2;
+    return table_in_lds<C>(epi) && stages < kTableBytes ? kTableBytes : stages;
 }
 
-template <int WM, int BK, int ST, int EPI>
-__global__ __launch_bounds__(256) void proj_kernel(ProjArgs a) {
-    constexpr int kStages = ST;
-    constexpr int kBK = BK;
-    constexpr int ROWB = BK * 2;      // bytes of one row of a stage
-    constexpr int NSL = BK / 8;       // 16-byte slots per row
+template <class C, int EPI>
+__global__ __launch_bounds__(C::WAVES * 64) __attribute__((amdgpu_waves_per_eu(C::WAVES / 4))) void proj_kernel(ProjArgs a) {
+    constexpr int kStages = C::ST;
+    constexpr int kBM = C::BM;
+    constexpr int kBK = C::BK;
+    constexpr int ROWB = kBK * 2;     // bytes of one row of a stage
+    constexpr int NSL = kBK / 8;      // 16-byte slots per row
     constexpr int RPC = 1024 / ROWB;  // rows per 1 KiB copy chunk
-    constexpr int SUB = BK / 16;      // MFMA k-steps per stage
-    constexpr int WAVES = 4;
-    constexpr int WR = kBM / WM;       // wavefronts along the rows
-    constexpr int WN = WAVES / WR;     // and along the tokens, 64 each
-    constexpr int BN = 64 * WN;
-    constexpr int MI = WM / 32;        // 32-row MFMA blocks per wavefront
+    constexpr int SUB = kBK / 16;     // MFMA k-steps per stage
+    constexpr int WAVES = C::WAVES;
+    constexpr int MI = C::MI, NJ = C::NJ;
+    constexpr int WM = 32 * MI, WT = 32 * NJ;  // rows and tokens of a wavefront
+    constexpr int WR = kBM / WM;      // wavefronts along the rows
+    constexpr int BN = C::BN;
+    static_assert(WR * (BN / WT) == WAVES && kBM % WM == 0 && BN % WT == 0, "wavefronts tile the workgroup");
     constexpr int NA = EPI == kSwiglu ? 2 : 1;
-    constexpr int A_BYTES = kBM * kBK * 2;  // one weight stage: 16 KiB
+    constexpr int A_BYTES = kBM * kBK * 2;  // one weight stage
     constexpr int B_BYTES = BN * kBK * 2;
     constexpr int A_CH = kBM / RPC / WAVES;   // 1 KiB copy chunks per wavefront
     constexpr int B_CH = BN / RPC / WAVES;
     constexpr int PER_STAGE = NA * A_CH + B_CH;  // copies per wavefront per k-step
     static_assert(A_CH >= 1 && B_CH >= 1 && PER_STAGE * (kStages - 2) <= 63, "copy plan");
-    static_assert((kStages - 1) * A_BYTES + kBM * ROWB <= 65536 && (kStages - 1) * B_BYTES + BN * ROWB <= 65536,
-                  "fragment reads reach every stage by immediate offsets");
-    __shared__ __align__(16) unsigned char lds[proj_lds_bytes(WM, BK, ST, EPI)];
+    __shared__ __align__(16) unsigned char lds[proj_lds_bytes<C>(EPI)];
     unsigned char *const a_lds = lds;                                  // [kStages][A_BYTES]
     unsigned char *const u_lds = lds + kStages * A_BYTES;              // SwiGLU up: [kStages][A_BYTES]
     unsigned char *const b_lds = lds + kStages * NA * A_BYTES;         // [kStages][B_BYTES]
@@ -120,25 +146,27 @@ __global__ __launch_bounds__(256) void proj_kernel(ProjArgs a) {
     const int h = lane >> 5;
 
     // XCD-aware tile: workgroup L runs on XCD L % 8; each XCD takes a
-    // contiguous slice of the tiles, ordered (row tile, token tile).
-    const int items = a.first_tile[a.segments] * a.n_tiles * a.ksplit;
+    // contiguous slice of the items, ordered (row tile, token tile, k split).
+    const int items = a.first_item[a.segments];
     const int per_xcd = (items + kXcds - 1) / kXcds;
     const int w_index = (int)(blockIdx.x % kXcds) * per_xcd + (int)(blockIdx.x / kXcds);
     if (w_index >= items) return;
-    const int t_index = w_index / a.ksplit, split = w_index % a.ksplit;
-    const int mt = t_index / a.n_tiles, nt = t_index % a.n_tiles;
     // The segment's matrix, by uniform selects (a dynamic index into the
     // kernel arguments would not stay scalar).
-    const bool s1 = a.segments > 1 && mt >= a.first_tile[1], s2 = a.segments > 2 && mt >= a.first_tile[2];
+    const bool s1 = a.segments > 1 && w_index >= a.first_item[1], s2 = a.segments > 2 && w_index >= a.first_item[2];
+    const int ksplit = s2 ? a.ksplit[2] : s1 ? a.ksplit[1] : a.ksplit[0];
+    const int in_seg = w_index - (s2 ? a.first_item[2] : s1 ? a.first_item[1] : 0);
+    const int t_index = in_seg / ksplit, split = in_seg % ksplit;
+    const int mt = t_index / a.n_tiles, nt = t_index % a.n_tiles;
     const int rows = s2 ? a.rows[2] : s1 ? a.rows[1] : a.rows[0];
-    const int m0 = (mt - (s2 ? a.first_tile[2] : s1 ? a.first_tile[1] : 0)) * kBM;
+    const int m0 = mt * kBM;
     const uint16_t *const wseg = s2 ? a.w[2] : s1 ? a.w[1] : a.w[0];
     uint16_t *const out = s2 ? a.out[2] : s1 ? a.out[1] : a.out[0];
     const int n0 = nt * BN;
     const int inner = a.inner;
     const int nk_all = inner / kBK;
-    const int kb = split * nk_all / a.ksplit;
-    const int nk = (split + 1) * nk_all / a.ksplit - kb;
+    const int kb = (int)((int64_t)split * nk_all / ksplit);
+    const int nk = (int)((int64_t)(split + 1) * nk_all / ksplit) - kb;
 
     // Copy offsets: chunk c of a stage is RPC rows; lane l lands in row
     // RPC c + l / NSL, physical slot l % NSL, and fetches the logical slot
@@ -171,18 +199,19 @@ __global__ __launch_bounds__(256) void proj_kernel(ProjArgs a) {
         u_dst[st] = EPI == kSwiglu ? lds_offset(u_lds + st * A_BYTES + wave * 1024) : 0;
         b_dst[st] = lds_offset(b_lds + st * B_BYTES + wave * 1024);
     }
-    auto copy_step = [&](int st, int kt) __attribute__((always_inline)) {
-        const int64_t k = (int64_t)kt * kBK * 2;
-#pragma unroll
-        for (int i = 0; i < A_CH; ++i) {
-            dma16_async(wbase + k, aoff[i], a_dst[st] + i * WAVES * 1024);
-            if (EPI == kSwiglu) dma16_async(ubase + k, aoff[i], u_dst[st] + i * WAVES * 1024);
+    // Copy c of a k-step into stage st, from byte offset k of its rows.
+    auto copy_one = [&](int st, int64_t k, int c) __attribute__((always_inline)) {
+        if (c < NA * A_CH) {
+            const int i = c / NA;
+            if (c % NA == 0) dma16_async(wbase + k, aoff[i], a_dst[st] + i * WAVES * 1024);
+            else dma16_async(ubase + k, aoff[i], u_dst[st] + i * WAVES * 1024);
+        } else {
+            const int i = c - NA * A_CH;
+            dma16_async(xbase + k, boff[i], b_dst[st] + i * WAVES * 1024);
         }
-#pragma unroll
-        for (int i = 0; i < B_CH; ++i) dma16_async(xbase + k, boff[i], b_dst[st] + i * WAVES * 1024);
     };
 
-    // Fragment addresses in stage 0: row WM wr + l % 32 (weights) or 64 wc +
+    // Fragment addresses in stage 0: row WM wr + l % 32 (weights) or WT wc +
     // l % 32 (tokens), logical slot 2 s + l / 32 of sub-step s, physical slot
     // that ^ proj_swz(row) = (2 s + h) ^ proj_swz(l % 32).  A 32-row block and
     // a stage are immediate offsets (the swizzle depends on row % 32 only).
@@ -194,42 +223,67 @@ __global__ __launch_bounds__(256) void proj_kernel(ProjArgs a) {
             const uint32_t sw = (uint32_t)(((2 * s + h) ^ proj_swz<NSL>(lane & 31)) * 16);
             fa[s] = abase + (uint32_t)(WM * wr + (lane & 31)) * ROWB + sw;
             fu[s] = ubase_l + (uint32_t)(WM * wr + (lane & 31)) * ROWB + sw;
-            fb[s] = bbase + (uint32_t)(64 * wc + (lane & 31)) * ROWB + sw;
+            fb[s] = bbase + (uint32_t)(WT * wc + (lane & 31)) * ROWB + sw;
         }
     }
 
-    floatx16_t acc[MI][2], accu[MI][2];
+    floatx16_t acc[MI][NJ], accu[MI][NJ];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 acc[i][j][r] = 0.0f;
                 if (EPI == kSwiglu) accu[i][j][r] = 0.0f;
             }
 
+    // Fragments of one sub-step: NJ of the tokens, MI of each weight matrix.
     struct Frag {
-        bf16x8_t a[MI], u[MI], b[2];
+        bf16x8_t a[NA * MI], b[NJ];
     };
-    auto read_frag = [&](Frag &f, int st, int s) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < MI; ++i) {
-            f.a[i] = lds_read_b128(fa[s] + st * A_BYTES + i * 32 * ROWB);
-            if (EPI == kSwiglu) f.u[i] = lds_read_b128(fu[s] + st * A_BYTES + i * 32 * ROWB);
+    constexpr int READS = NA * MI + NJ;
+    constexpr int MFMAS = NA * MI * NJ;
+    auto read_one = [&](Frag &f, int st, int s, int r) __attribute__((always_inline)) {
+        // the first MFMA needs a[0] and b[0]
+        if (r == 0) f.b[0] = lds_read_b128(fb[s] + st * B_BYTES);
+        else if (r <= NA * MI) {
+            const int i = (r - 1) / NA;
+            if ((r - 1) % NA == 0) f.a[NA * i] = lds_read_b128(fa[s] + st * A_BYTES + i * 32 * ROWB);
+            else f.a[NA * i + 1] = lds_read_b128(fu[s] + st * A_BYTES + i * 32 * ROWB);
+        } else {
+            const int j = r - NA * MI;
+            f.b[j] = lds_read_b128(fb[s] + st * B_BYTES + j * 32 * ROWB);
         }
-#pragma unroll
-        for (int j = 0; j < 2; ++j) f.b[j] = lds_read_b128(fb[s] + st * B_BYTES + j * 32 * ROWB);
     };
-    auto mfma = [&](const Frag &f) __attribute__((always_inline)) {
+    auto mfma_one = [&](const Frag &f, int m) __attribute__((always_inline)) {
+        const int j = m / (NA * MI), i = m % (NA * MI) / NA;
+        if (m % NA == 0) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[NA * i], f.b[j], acc[i][j], 0, 0, 0);
+        else accu[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[NA * i + 1], f.b[j], accu[i][j], 0, 0, 0);
+    };
+    // One phase: the MFMAs of `cur`, with the fragment reads of sub-step s of
+    // stage st into `nxt` spread over the first half of them and part `part`
+    // of SUB of the k-step's copies into stage sd over all of them.  The order is pinned: left to
+    // itself the compiler sinks the reads below the MFMAs, and with one
+    // wavefront per SIMD every phase then waits out their latency.
+    auto phase = [&](const Frag &cur, Frag &nxt, int st, int s, auto mfma_tag, auto read_tag, int part, int sd,
+                     int64_t k) __attribute__((always_inline)) {
+        constexpr bool do_mfma = decltype(mfma_tag)::value, do_read = decltype(read_tag)::value;
+        constexpr int HALF = MFMAS >= 2 ? MFMAS / 2 : 1;
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
+        for (int m = 0; m < MFMAS; ++m) {
+            if constexpr (do_read) {
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[i], f.b[j], acc[i][j], 0, 0, 0);
-                if (EPI == kSwiglu)
-                    accu[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.u[i], f.b[j], accu[i][j], 0, 0, 0);
+                for (int r = 0; r < READS; ++r)
+                    if (r * HALF / READS == m) read_one(nxt, st, s, r);
             }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (do_mfma) mfma_one(cur, m);
+#pragma unroll
+            for (int c = 0; c < PER_STAGE; ++c)
+                if (c * (SUB * MFMAS) / PER_STAGE == part * MFMAS + m) copy_one(sd, k, c);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
 
     // K loop.  Iteration kt: this wavefront's copy of k-step kt has landed
@@ -237,46 +291,46 @@ __global__ __launch_bounds__(256) void proj_kernel(ProjArgs a) {
     // stage of kt-1, which receives k-step kt + kStages - 1 (the last k-step
     // is repeated past the end so the wait counts stay exact).  The fragments
     // of kt-1's last sub-step were read before the barrier; their MFMAs run
-    // while the first fragments of kt are in flight.
-    Frag cur, nxt;
-#pragma unroll
-    for (int st = 0; st < kStages - 1; ++st) copy_step(st, min(st, nk - 1));
-    auto iteration = [&](int kt, int st, int sd, auto first_tag) __attribute__((always_inline)) {
-        constexpr bool first = decltype(first_tag)::value;
-        __builtin_amdgcn_s_waitcnt(vmcnt_lds_imm((kStages - 2) * PER_STAGE));
-        raw_barrier();
-        read_frag(nxt, st, 0);
-        if constexpr (!first) mfma(cur);
-        copy_step(sd, min(kt + kStages - 1, nk - 1));
-#pragma unroll
-        for (int s = 0; s < SUB; ++s) {
-            __builtin_amdgcn_sched_barrier(0);
-            cur = nxt;
-            if (s + 1 < SUB) read_frag(nxt, st, s + 1);
-            if (s + 1 < SUB) mfma(cur);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
+    // while the first fragments of kt are in flight.  Sub-step s uses
+    // fragment set s % 2.
     using Yes = std::true_type;
     using No = std::false_type;
+    static_assert(SUB % 2 == 0, "sub-steps alternate two fragment sets");
+    Frag f0, f1;
+    auto k_bytes = [&](int kt) __attribute__((always_inline)) { return (int64_t)min(kt, nk - 1) * ROWB; };
+#pragma unroll
+    for (int st = 0; st < kStages - 1; ++st)
+#pragma unroll
+        for (int c = 0; c < PER_STAGE; ++c) copy_one(st, k_bytes(st), c);
+    auto iteration = [&](int kt, int st, int sd, auto mfma_tag) __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(vmcnt_lds_imm((kStages - 2) * PER_STAGE));
+        raw_barrier();
+        const int64_t k = k_bytes(kt + kStages - 1);
+        phase(f1, f0, st, 0, mfma_tag, Yes{}, 0, sd, k);
+#pragma unroll
+        for (int s = 0; s + 1 < SUB; ++s) {
+            if (s % 2 == 0) phase(f0, f1, st, s + 1, Yes{}, Yes{}, s + 1, sd, k);
+            else phase(f1, f0, st, s + 1, Yes{}, Yes{}, s + 1, sd, k);
+        }
+    };
     // Stage of k-step kt is kt % kStages; the loop is unrolled by kStages so
     // every stage index is a constant.
-    iteration(0, 0, kStages - 1, Yes{});
+    iteration(0, 0, kStages - 1, No{});
     for (int kt = 1; kt < nk; kt += kStages) {
 #pragma unroll
         for (int u = 0; u < kStages; ++u) {
             if (kt + u >= nk) break;
-            iteration(kt + u, (1 + u) % kStages, u % kStages, No{});
+            iteration(kt + u, (1 + u) % kStages, u % kStages, Yes{});
         }
     }
-    mfma(cur);
+    phase(f1, f0, 0, 0, Yes{}, No{}, SUB, 0, 0);
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // no copy may still target LDS at exit
 
     // SwiGLU: the activation table replaces the stages in LDS (one 128 KiB
     // copy per workgroup, from L2), after every wavefront's last fragment
     // read.
-    const uint16_t *table = nullptr;
-    if constexpr (EPI == kSwiglu) {
+    const uint16_t *table = a.act_table;
+    if (table_in_lds<C>(EPI) && ksplit == 1) {
         __syncthreads();
         const char *tb = uniform_ptr(reinterpret_cast<const char *>(a.act_table));
         const uint32_t dst = lds_offset(lds + wave * 1024);
@@ -288,16 +342,16 @@ __global__ __launch_bounds__(256) void proj_kernel(ProjArgs a) {
         table = reinterpret_cast<const uint16_t *>(lds);
     }
 
-    // Epilogue: lane l holds token 64 wc + 32 j + l % 32 and, per group g of
+    // Epilogue: lane l holds token WT wc + 32 j + l % 32 and, per group g of
     // four accumulators, rows WM wr + 32 i + 8 g + 4 h .. +3.
-    if (a.ksplit > 1) {
-        const int64_t obase = s2 ? a.out_base[2] : s1 ? a.out_base[1] : 0;
-        float *const part = a.partial + (int64_t)split * NA * a.out_base[a.segments] + obase;
-        float *const part_up = part + a.out_base[a.segments];
-        const bool vecf = (rows & 3) == 0 && (obase & 3) == 0;
+    if (ksplit > 1) {
+        const int64_t outs = (int64_t)a.tokens * rows;
+        float *const part = a.partial + (s2 ? a.part_base[2] : s1 ? a.part_base[1] : a.part_base[0]) + split * NA * outs;
+        float *const part_up = part + outs;
+        const bool vecf = (rows & 3) == 0;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int t = n0 + 64 * wc + 32 * j + (lane & 31);
+        for (int j = 0; j < NJ; ++j) {
+            const int t = n0 + WT * wc + 32 * j + (lane & 31);
             if (t >= a.tokens) continue;
 #pragma unroll
             for (int i = 0; i < MI; ++i)
@@ -316,7 +370,9 @@ __global__ __launch_bounds__(256) void proj_kernel(ProjArgs a) {
                             *reinterpret_cast<floatx4_t *>(part_up + o) = u;
                         }
                     } else {
-                        for (int e = 0; e < 4 && r + e < rows; ++e) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            if (r + e >= rows) break;
                             part[o + e] = acc[i][j][4 * g + e];
                             if (EPI == kSwiglu) part_up[o + e] = accu[i][j][4 * g + e];
                         }
@@ -328,8 +384,8 @@ __global__ __launch_bounds__(256) void proj_kernel(ProjArgs a) {
     const bool vec = (rows & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0 &&
                      (EPI != kAdd || (reinterpret_cast<uintptr_t>(a.resid) & 7) == 0);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int t = n0 + 64 * wc + 32 * j + (lane & 31);
+    for (int j = 0; j < NJ; ++j) {
+        const int t = n0 + WT * wc + 32 * j + (lane & 31);
         if (t >= a.tokens) continue;
 #pragma unroll
         for (int i = 0; i < MI; ++i)
@@ -370,37 +426,39 @@ __global__ __launch_bounds__(256) void proj_kernel(ProjArgs a) {
     }
 }
 
-// Split launches: out = epilogue(BF16(partial[0] + partial[1] + ...)), the
-// partials added in split order, four outputs per thread.
+// Split segments (grid y): out = epilogue(BF16(partial[0] + partial[1] +
+// ...)), the partials added in split order, four outputs per thread.
 template <int EPI>
 __global__ __launch_bounds__(256) void proj_merge_kernel(ProjArgs a) {
     constexpr int NA = EPI == kSwiglu ? 2 : 1;
-    const int64_t n = a.out_base[a.segments];
+    const int seg = blockIdx.y;
+    const int ksplit = a.ksplit[seg];
+    const int64_t n = (int64_t)a.tokens * a.rows[seg];
     const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (i0 >= n) return;
-    // Four outputs of one segment with 16-byte partials and 8-byte outputs
-    // (and residual): one vector access each; otherwise element by element.
-    // The arithmetic per element is the same either way.
-    const int seg0 = (a.segments > 2 && i0 >= a.out_base[2]) ? 2 : (a.segments > 1 && i0 >= a.out_base[1]) ? 1 : 0;
-    const int64_t li0 = i0 - a.out_base[seg0];
-    const bool vec = i0 + 3 < a.out_base[seg0 + 1] && (li0 & 3) == 0 &&
-                     ((reinterpret_cast<uintptr_t>(a.partial) | reinterpret_cast<uintptr_t>(a.out[seg0]) |
-                       (EPI == kAdd ? reinterpret_cast<uintptr_t>(a.resid) : 0)) & 15) == 0;
+    if (ksplit == 1 || i0 >= n) return;
+    const float *const part = a.partial + a.part_base[seg];
+    uint16_t *const out = a.out[seg];
+    // Four outputs with 16-byte partials and 8-byte outputs (and residual):
+    // one vector access each; otherwise element by element.  The arithmetic
+    // per element is the same either way.
+    const bool vec = (n & 3) == 0 && (reinterpret_cast<uintptr_t>(part) & 15) == 0 &&
+                     ((reinterpret_cast<uintptr_t>(out) | (EPI == kAdd ? reinterpret_cast<uintptr_t>(a.resid) : 0)) & 7) == 0;
     if (vec) {
-        float4 v = *reinterpret_cast<const float4 *>(a.partial + i0);
-        float4 vu = EPI == kSwiglu ? *reinterpret_cast<const float4 *>(a.partial + n + i0) : float4{};
-        for (int s = 1; s < a.ksplit; ++s) {
-            const float4 w = *reinterpret_cast<const float4 *>(a.partial + (int64_t)s * NA * n + i0);
+        float4 v = *reinterpret_cast<const float4 *>(part + i0);
+        float4 vu = EPI == kSwiglu ? *reinterpret_cast<const float4 *>(part + n + i0) : float4{};
+#pragma unroll 4
+        for (int s = 1; s < ksplit; ++s) {
+            const float4 w = *reinterpret_cast<const float4 *>(part + (int64_t)s * NA * n + i0);
             v = float4{__fadd_rn(v.x, w.x), __fadd_rn(v.y, w.y), __fadd_rn(v.z, w.z), __fadd_rn(v.w, w.w)};
             if (EPI == kSwiglu) {
-                const float4 wu = *reinterpret_cast<const float4 *>(a.partial + ((int64_t)s * NA + 1) * n + i0);
+                const float4 wu = *reinterpret_cast<const float4 *>(part + ((int64_t)s * NA + 1) * n + i0);
                 vu = float4{__fadd_rn(vu.x, wu.x), __fadd_rn(vu.y, wu.y), __fadd_rn(vu.z, wu.z), __fadd_rn(vu.w, wu.w)};
             }
         }
         const float vs[4] = {v.x, v.y, v.z, v.w}, us[4] = {vu.x, vu.y, vu.z, vu.w};
         uint16_t rs[4] = {0, 0, 0, 0};
         if (EPI == kAdd) {
-            const uint2 r = *reinterpret_cast<const uint2 *>(a.resid + li0);
+            const uint2 r = *reinterpret_cast<const uint2 *>(a.resid + i0);
             rs[0] = (uint16_t)r.x; rs[1] = (uint16_t)(r.x >> 16); rs[2] = (uint16_t)r.y; rs[3] = (uint16_t)(r.y >> 16);
         }
         uint16_t ys[4];
@@ -411,7 +469,7 @@ __global__ __launch_bounds__(256) void proj_merge_kernel(ProjArgs a) {
             if (EPI == kAdd) y = write_bf16(__fadd_rn(read_bf16(rs[e]), read_bf16(y)));
             ys[e] = y;
         }
-        *reinterpret_cast<uint2 *>(a.out[seg0] + li0) =
+        *reinterpret_cast<uint2 *>(out + i0) =
             uint2{(uint32_t)ys[0] | ((uint32_t)ys[1] << 16), (uint32_t)ys[2] | ((uint32_t)ys[3] << 16)};
         return;
     }
@@ -419,17 +477,15 @@ __global__ __launch_bounds__(256) void proj_merge_kernel(ProjArgs a) {
     for (int e = 0; e < 4; ++e) {
         const int64_t i = i0 + e;
         if (i >= n) break;
-        float v = a.partial[i], vu = EPI == kSwiglu ? a.partial[n + i] : 0.0f;
-        for (int s = 1; s < a.ksplit; ++s) {
-            v = __fadd_rn(v, a.partial[(int64_t)s * NA * n + i]);
-            if (EPI == kSwiglu) vu = __fadd_rn(vu, a.partial[((int64_t)s * NA + 1) * n + i]);
+        float v = part[i], vu = EPI == kSwiglu ? part[n + i] : 0.0f;
+        for (int s = 1; s < ksplit; ++s) {
+            v = __fadd_rn(v, part[(int64_t)s * NA * n + i]);
+            if (EPI == kSwiglu) vu = __fadd_rn(vu, part[((int64_t)s * NA + 1) * n + i]);
         }
-        const int seg = (a.segments > 2 && i >= a.out_base[2]) ? 2 : (a.segments > 1 && i >= a.out_base[1]) ? 1 : 0;
-        const int64_t li = i - a.out_base[seg];
         uint16_t y = write_bf16(v);
         if (EPI == kSwiglu) y = swiglu_mul_bf16(a.act_table[y], write_bf16(vu));
-        if (EPI == kAdd) y = write_bf16(__fadd_rn(read_bf16(a.resid[li]), read_bf16(y)));
-        a.out[seg][li] = y;
+        if (EPI == kAdd) y = write_bf16(__fadd_rn(read_bf16(a.resid[i]), read_bf16(y)));
+        out[i] = y;
     }
 }
 
@@ -475,64 +531,171 @@ __global__ __launch_bounds__(256) void proj_generic_kernel(ProjArgs a) {
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// The configurations, smallest tile first; a SwiGLU tile holds half the output
+// rows (gate and up rows side by side).  Wavefront tiles of 32 x 32 to 64 x 64,
+// two wavefronts per SIMD except in the smallest, which fits twice on a CU.
+enum { kTile64x64, kTile64x128, kTile128x128, kTile128x256, kTiles };
+template <int TILE, int EPI>
+struct TileConfig;
+template <int EPI>
+struct TileConfig<kTile64x64, EPI> : Config<64, 64, 1, 1, 64, 4, 4> {};
+template <int EPI>
+struct TileConfig<kTile64x128, EPI> : Config<64, 128, 1, 1, 64, EPI == kSwiglu ? 3 : 4, 8> {};
+template <int EPI>
+struct TileConfig<kTile128x128, EPI> : Config<128, 128, 1, 2, 64, EPI == kSwiglu ? 3 : 4, 8> {};
+template <int EPI>
+struct TileConfig<kTile128x256, EPI>
+    : Config<EPI == kSwiglu ? 64 : 128, 256, EPI == kSwiglu ? 1 : 2, 2, 64, 3, 8> {};
+
+// What the choices below know of a configuration: its tile, and the measured
+// time of a k-step of 64 inputs with one workgroup per CU and the weights in
+// HBM (us; two resident 64 x 64 workgroups take twice that).
+struct TileCost {
+    int bm, bn;
+    double step;
+};
+constexpr TileCost kPlainCost[kTiles] = {{64, 64, 0.27}, {64, 128, 0.36}, {128, 128, 0.50}, {128, 256, 0.71}};
+constexpr TileCost kSwigluCost[kTiles] = {{64, 64, 0.62}, {64, 128, 0.55}, {128, 128, 1.00}, {64, 256, 0.80}};
+constexpr int kCus = 256;
+constexpr double kStreamBytesPerUs = 4.8e6;   // weights from HBM
+constexpr double kMergeUs = 3.5;              // the merge launch, beside its traffic
+constexpr double kMergeBytesPerUs = 6.0e6;
+constexpr int kMinSplitSteps = 8;             // k-steps of a split, at least
+constexpr int64_t kSplitBytes = 16ll << 20;   // partials of one product's sum, at most (inner < 8192)
+constexpr double kGain = 0.5;                 // a larger tile or split must save this (us)
+
+int64_t tiles_of(const TileCost &c, int rows, int tokens) {
+    return (int64_t)((rows + c.bm - 1) / c.bm) * ((tokens + c.bn - 1) / c.bn);
+}
+
+double split_cost(int ksplit, int64_t outputs) {
+    return ksplit == 1 ? 0.0 : kMergeUs + 2.0 * ksplit * outputs * sizeof(float) / kMergeBytesPerUs;
+}
+
+// K splits of the product of a [rows][inner] matrix with `tokens` rows: the
+// count, on its best configuration, of the least predicted time.  It depends
+// on the product's own shape only, never on the launch the product is part
+// of, so every entry point (one matrix or several, fused epilogue or not) sums
+// a given product in the same order.  A narrow matrix counts as a square one:
+// it is a K or V beside its Q, whose splits leave the launch one wave of
+// workgroups, while splits of its own put more items behind them (Q, K, V of
+// 4,096 + 1,024 + 1,024 rows at 128 tokens: 20.9 us with Q's four splits for
+// all, 31.4 us with eight for K and V).
+int product_ksplit(int inner, int rows, int tokens) {
+    if (inner < 8192) rows = std::max(rows, std::min(inner, 4096));
+    const int steps = inner / kKAlign;
+    const double stream = (double)rows * inner * 2 / kStreamBytesPerUs;
+    const int64_t outputs = (int64_t)rows * tokens;
+    int best = 1;
+    double least = 0.0;
+    for (int k = 1; k <= 8; k *= 2) {
+        if (k > 1 && (steps / k < kMinSplitSteps ||
+                      (inner < 8192 && (int64_t)k * outputs * (int64_t)sizeof(float) > kSplitBytes)))
+            break;
+        double us = 0.0;
+        for (int t = 0; t < kTiles; ++t) {
+            const TileCost &c = kPlainCost[t];
+            const int64_t rounds = (tiles_of(c, rows, tokens) * k + kCus - 1) / kCus;
+            const double busy = rounds * ((steps + k - 1) / k) * c.step;
+            if (t == 0 || busy < us) us = busy;
+        }
+        us = std::max(us, stream) + split_cost(k, outputs);
+        if (k == 1 || us < least - kGain) {
+            least = us;
+            best = k;
+        }
+    }
+    return best;
+}
+
+// Configuration of a launch, given its products' splits: the one that
+// finishes first when its items are dealt to the resident workgroups.  Which
+// one it is changes no bit of the results.
+int choose_tile(const ProjArgs &a, bool swiglu) {
+    const int steps = a.inner / kKAlign;
+    int best = 0;
+    double least = 0.0;
+    for (int t = 0; t < kTiles; ++t) {
+        const TileCost &c = swiglu ? kSwigluCost[t] : kPlainCost[t];
+        int64_t items = 0;
+        double work = 0.0, longest = 0.0, bytes = 0.0;  // work and longest in k-steps
+        for (int s = 0; s < a.segments; ++s) {
+            const int64_t n = tiles_of(c, a.rows[s], a.tokens) * a.ksplit[s];
+            const double each = (double)steps / a.ksplit[s];
+            items += n;
+            work += n * each;
+            longest = std::max(longest, each);
+            bytes += (double)a.rows[s] * a.inner * 2 * (swiglu ? 2 : 1);
+        }
+        // equal items run in whole rounds; unequal ones leave about half of
+        // the longest item behind the mean
+        const double rounds = (double)((items + kCus - 1) / kCus);
+        const bool equal = work == items * longest;
+        const double span = equal ? rounds * longest : std::max(longest, work / kCus + (rounds > 1 ? longest / 2 : 0.0));
+        const double us = std::max(span * c.step, bytes / kStreamBytesPerUs);
+        if (t == 0 || us < least - kGain) {
+            least = us;
+            best = t;
+        }
+    }
+    return best;
+}
+
 }  // namespace
 
-// A long inner dimension (the down projection's 14,336) leaves too few
-// 128 x 128 output tiles to fill the CUs at prompt-chunk sizes; its k range is
-// split in two, with a merge launch.  The choice depends on inner only, so
-// every entry point (one matrix or several, fused epilogue or not) sums a
-// given product in the same order.
-int proj_ksplit(int inner) { return inner >= 8192 && inner % (2 * kKAlign) == 0 ? 2 : 1; }
+size_t proj_partial_floats(const int *rows, int count, int products, int inner, int tokens) {
+    size_t total = 0;
+    for (int s = 0; s < count; ++s) {
+        const int k = product_ksplit(inner, rows[s], tokens);
+        if (k > 1) total += ((size_t)k * products * rows[s] * tokens + 3) & ~(size_t)3;
+    }
+    return total;
+}
 
 namespace {
 
+template <class C, int EPI>
+hipError_t launch_config(ProjArgs &a, hipStream_t stream) {
+    a.n_tiles = (a.tokens + C::BN - 1) / C::BN;
+    a.first_item[0] = 0;
+    for (int s = 0; s < a.segments; ++s)
+        a.first_item[s + 1] = a.first_item[s] + (a.rows[s] + C::BM - 1) / C::BM * a.n_tiles * a.ksplit[s];
+    for (int s = a.segments + 1; s <= kMaxSeg; ++s) a.first_item[s] = a.first_item[a.segments];
+    const unsigned grid = (unsigned)((a.first_item[a.segments] + kXcds - 1) / kXcds * kXcds);
+    hipLaunchKernelGGL((proj_kernel<C, EPI>), dim3(grid), dim3(C::WAVES * 64), 0, stream, a);
+    return hipGetLastError();
+}
+
 template <int EPI>
 hipError_t launch(ProjArgs &a, hipStream_t stream) {
-    a.first_tile[0] = 0;
-    for (int s = 0; s < a.segments; ++s) a.first_tile[s + 1] = a.first_tile[s] + (a.rows[s] + kBM - 1) / kBM;
-    for (int s = a.segments + 1; s <= kMaxSeg; ++s) a.first_tile[s] = a.first_tile[a.segments];
     bool fast = a.inner % kKAlign == 0 && aligned16(a.x) && (EPI != kSwiglu || aligned16(a.w_up));
     for (int s = 0; s < a.segments; ++s) fast = fast && aligned16(a.w[s]);
     if (!fast) {
-        a.ksplit = 1;
         int64_t total = 0;
         for (int s = 0; s < a.segments; ++s) total += (int64_t)a.rows[s] * a.tokens;
         hipLaunchKernelGGL((proj_generic_kernel<EPI>), dim3((unsigned)((total + 3) / 4)), dim3(256), 0, stream, a);
         return hipGetLastError();
     }
-    // 128 x 128 tiles (64 x 64 per wavefront) when the launch has at least
-    // three of them per four CUs, 128 x 64 (32 x 64 per wavefront) below.
-    // Measured on the cfg5 shapes at 512 tokens (us, 128 x 128 / 128 x 64):
-    // Q, K, V 33.4 / 36.7; O 36.9 / 26.0; gate and up 151 / 215; down 137 /
-    // 107 (a k-step of 128 with two stages was slower for every shape).
-    const int64_t m_tiles = a.first_tile[a.segments];
-    a.ksplit = proj_ksplit(a.inner);
-    if (a.ksplit > 1 && !a.partial) return hipErrorInvalidValue;
-    a.out_base[0] = 0;
-    for (int s = 0; s < a.segments; ++s) a.out_base[s + 1] = a.out_base[s] + (int64_t)a.rows[s] * a.tokens;
-    for (int s = a.segments + 1; s <= kMaxSeg; ++s) a.out_base[s] = a.out_base[a.segments];
-    const bool wide = (a.ksplit > 1 || m_tiles * ((a.tokens + 127) / 128) >= 192) &&
-                      proj_lds_bytes(64, kBK, kStages, EPI) <= 163840;
-    const int bn = wide ? 128 : 64;
-    a.n_tiles = (a.tokens + bn - 1) / bn;
-    const int64_t tiles = m_tiles * a.n_tiles * a.ksplit;
-    const unsigned grid = (unsigned)(((tiles + kXcds - 1) / kXcds) * kXcds);
-    if constexpr (proj_lds_bytes(64, kBK, kStages, EPI) <= 163840) {
-        if (wide) {
-            hipLaunchKernelGGL((proj_kernel<64, kBK, kStages, EPI>), dim3(grid), dim3(256), 0, stream, a);
-            return hipGetLastError();
-        }
+    constexpr int products = EPI == kSwiglu ? 2 : 1;
+    int64_t base = 0, most = 0;
+    for (int s = 0; s < a.segments; ++s) {
+        a.ksplit[s] = product_ksplit(a.inner, a.rows[s], a.tokens);
+        a.part_base[s] = base;
+        if (a.ksplit[s] == 1) continue;
+        if (!a.partial) return hipErrorInvalidValue;
+        base += ((int64_t)a.ksplit[s] * products * a.rows[s] * a.tokens + 3) & ~(int64_t)3;
+        most = std::max(most, (int64_t)a.rows[s] * a.tokens);
     }
-    hipLaunchKernelGGL((proj_kernel<32, kBK, kStages, EPI>), dim3(grid), dim3(256), 0, stream, a);
-    return hipGetLastError();
-}
-
-template <int EPI>
-hipError_t launch_split(ProjArgs &a, hipStream_t stream) {
-    if (hipError_t e = launch<EPI>(a, stream)) return e;
-    if (a.ksplit < 2) return hipSuccess;
-    const int64_t n = a.out_base[a.segments];
-    hipLaunchKernelGGL((proj_merge_kernel<EPI>), dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, stream, a);
+    hipError_t e;
+    switch (choose_tile(a, EPI == kSwiglu)) {
+        case kTile64x64: e = launch_config<TileConfig<kTile64x64, EPI>, EPI>(a, stream); break;
+        case kTile64x128: e = launch_config<TileConfig<kTile64x128, EPI>, EPI>(a, stream); break;
+        case kTile128x128: e = launch_config<TileConfig<kTile128x128, EPI>, EPI>(a, stream); break;
+        default: e = launch_config<TileConfig<kTile128x256, EPI>, EPI>(a, stream); break;
+    }
+    if (e != hipSuccess || !most) return e;
+    hipLaunchKernelGGL((proj_merge_kernel<EPI>), dim3((unsigned)((most + 1023) / 1024), (unsigned)a.segments), dim3(256),
+                       0, stream, a);
     return hipGetLastError();
 }
 
@@ -551,7 +714,7 @@ hipError_t launch_proj(const SkinnyMatrix *m, int count, const uint16_t *x, int 
     a.inner = inner;
     a.tokens = tokens;
     a.partial = partial;
-    return launch_split<kPlain>(a, stream);
+    return launch<kPlain>(a, stream);
 }
 
 hipError_t launch_proj_add(const SkinnyMatrix &m, const uint16_t *resid, const uint16_t *x, int inner, int tokens,
@@ -566,7 +729,7 @@ hipError_t launch_proj_add(const SkinnyMatrix &m, const uint16_t *resid, const u
     a.inner = inner;
     a.tokens = tokens;
     a.partial = partial;
-    return launch_split<kAdd>(a, stream);
+    return launch<kAdd>(a, stream);
 }
 
 hipError_t launch_proj_swiglu(const uint16_t *w_gate, const uint16_t *w_up, uint16_t *out, int rows,
@@ -583,7 +746,7 @@ hipError_t launch_proj_swiglu(const uint16_t *w_gate, const uint16_t *w_up, uint
     a.inner = inner;
     a.tokens = tokens;
     a.partial = partial;
-    return launch_split<kSwiglu>(a, stream);
+    return launch<kSwiglu>(a, stream);
 }
 
 }  // namespace mslim
