@@ -196,19 +196,12 @@ void decode_place_partials(mslim::DecodeLaunch &l, void *base) {
     l.partial_acc = reinterpret_cast<float *>(static_cast<char *>(base) + ml_bytes);
 }
 
-int decode_common(Context &c, mslim::DecodeLaunch &l, const int32_t *seq_lens, int split_tokens) {
-    if (int rc = decode_prepare(l, seq_lens, split_tokens)) return rc;
-    if (int rc = grow_device(c, &c.workspace, &c.workspace_bytes, mslim::decode_partial_bytes(l),
-                             "hipMalloc decode split workspace"))
-        return rc;
-    decode_place_partials(l, c.workspace);
-    // One split counter per (sequence, kv head); the kernel leaves them at
-    // zero, so they are cleared only when the buffer is (re)allocated.
-    const size_t ctr_bytes = (size_t)std::max(l.batch, mslim::kInlineBatch) * l.kv_heads * sizeof(int);
-    if (c.counter_bytes < ctr_bytes) {
+// At least n split counters in the context.  The kernels leave them at zero,
+// so they are cleared only when the buffer is (re)allocated or a launch failed.
+int split_counters(Context &c, size_t n) {
+    if (c.counter_bytes < n * sizeof(int)) {
         void *mem = c.counters;
-        if (int rc = grow_device(c, &mem, &c.counter_bytes, ctr_bytes, "hipMalloc decode split counters"))
-            return rc;
+        if (int rc = grow_device(c, &mem, &c.counter_bytes, n * sizeof(int), "hipMalloc split counters")) return rc;
         c.counters = static_cast<int *>(mem);
         c.counters_dirty = true;
     }
@@ -219,6 +212,17 @@ int decode_common(Context &c, mslim::DecodeLaunch &l, const int32_t *seq_lens, i
             return rc;
         c.counters_dirty = false;
     }
+    return 0;
+}
+
+int decode_common(Context &c, mslim::DecodeLaunch &l, const int32_t *seq_lens, int split_tokens) {
+    if (int rc = decode_prepare(l, seq_lens, split_tokens)) return rc;
+    if (int rc = grow_device(c, &c.workspace, &c.workspace_bytes, mslim::decode_partial_bytes(l),
+                             "hipMalloc decode split workspace"))
+        return rc;
+    decode_place_partials(l, c.workspace);
+    // One split counter per (sequence, kv head).
+    if (int rc = split_counters(c, (size_t)std::max(l.batch, mslim::kInlineBatch) * l.kv_heads)) return rc;
     l.counters = c.counters;
     l.separate_merge = c.separate_merge;
     mslim::DecodeTables tables{};
@@ -269,7 +273,7 @@ size_t format_bytes(int format) { return format == MSLIM_ATTN_FORMAT_F32 ? 4 : 2
 int frames_enqueue(Context &c, mslim::FramesLaunch &l, uint64_t *scratch) {
     *scratch = 0;
     l.scale = (float)(1.0 / std::sqrt((double)l.head_dim));
-    l.split_tokens = l.tokens > 0 ? mslim::frames_split_tokens(l.tokens, l.q_heads) : 256;
+    l.split_tokens = l.tokens > 0 ? mslim::frames_split_tokens(l) : 256;
     const int64_t splits = (l.tokens + l.split_tokens - 1) / l.split_tokens;
     if (splits > 1) {
         const size_t ml = (size_t)l.q_heads * splits * 2 * sizeof(float);
@@ -280,8 +284,14 @@ int frames_enqueue(Context &c, mslim::FramesLaunch &l, uint64_t *scratch) {
         l.partial_ml = static_cast<float *>(c.workspace);
         l.partial_acc = reinterpret_cast<float *>(static_cast<char *>(c.workspace) + ml);
         *scratch = ml + acc;
+        if (mslim::frames_grouped(l)) {
+            if (int rc = split_counters(c, mslim::frames_counters(l))) return rc;
+            l.counters = c.counters;
+        }
     }
-    return check_hip(mslim::launch_frames_decode(l, c.stream), "frames decode launch");
+    const int rc = check_hip(mslim::launch_frames_decode(l, c.stream), "frames decode launch");
+    if (rc && l.counters) c.counters_dirty = true;
+    return rc;
 }
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }

@@ -114,11 +114,16 @@ struct FramesLaunch {
     float *partial_ml, *partial_acc;  // [q_heads][splits][2], [q_heads][splits][D]
     int64_t tokens;                   // >= 1
     int q_heads, kv_heads, head_dim;
-    int split_tokens;                 // multiple of 256
+    int split_tokens;                 // of frames_split_tokens
     float scale;
+    int *counters;                    // frames_counters() ints, zero between launches, when frames_grouped
 };
-// Tokens per split for a launch of `tokens` tokens and q_heads heads.
-int frames_split_tokens(int64_t tokens, int q_heads);
+// True when the kernel that shares K and V over a group of query heads covers
+// this launch; it merges its splits itself, through the counters.
+bool frames_grouped(const FramesLaunch &l);
+int frames_counters(const FramesLaunch &l);
+// Tokens per split of a launch.
+int frames_split_tokens(const FramesLaunch &l);
 hipError_t launch_frames_decode(const FramesLaunch &l, hipStream_t stream);
 
 hipError_t launch_rmsnorm(const uint16_t *in, const uint16_t *w, uint16_t *out, int tokens,
