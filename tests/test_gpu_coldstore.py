@@ -154,3 +154,36 @@ def test_cfg4_layer_seal_properties(ctx):
         page_id, token_start, layer, tokens, pool_page = descs[i]
         got = file_bytes(f[i], k_host, v_host, pool_page, tokens)
         assert got == oracle_record(k_host, v_host, page_id, token_start, layer, tokens, pool_page, 16)
+
+
+@pytest.mark.parametrize("kv_heads,head_dim,page_tokens", [(8, 128, 32), (3, 72, 16), (1, 8, 64)])
+def test_every_token_count_in_one_launch(ctx, kv_heads, head_dim, page_tokens):
+    # every record length of a page side by side (messages that end, and
+    # payloads that start, at every place of a 64-byte block; payloads on both
+    # sides of the checksum kernel's 32 KiB tile), records that start inside a
+    # page, one invalid record among them, and a workgroup that is not full
+    rng = np.random.default_rng(page_tokens)
+    pool_pages = 7
+    k, v = make_pool(rng, pool_pages, kv_heads, page_tokens, head_dim)
+    records = [(t, 0) for t in range(1, page_tokens + 1)] + [(t, page_tokens - t) for t in range(1, page_tokens, 5)]
+    records.insert(5, (page_tokens + 1, 0))  # invalid
+    records += [(page_tokens, 0)] * (70 - len(records) % 64)
+    arr = (mslim_attn.PageRecord * len(records))()
+    for i, (tokens, first) in enumerate(records):
+        arr[i] = mslim_attn.PageRecord(i + 1, 100 * i, i % 5, tokens, i % pool_pages, first)
+    slot = mslim_attn.Context.record_frame_bytes(page_tokens)
+    frames = torch.full((len(records) * slot,), 0xAB, dtype=torch.uint8, device="cuda")
+    ctx.record_frames(device(k), device(v), pool_pages, page_tokens, kv_heads, head_dim, 1,
+                      device(np.frombuffer(bytes(arr), np.uint8)), len(records), frames)
+    torch.cuda.synchronize()
+    frames = frames.cpu().numpy()
+    for i, (tokens, first) in enumerate(records):
+        frame = frames[i * slot:(i + 1) * slot]
+        if tokens > page_tokens:
+            assert not frame.any()
+            continue
+        kp, vp = (np.ascontiguousarray(x[i % pool_pages, :, first:first + tokens, :]).view(np.uint8).tobytes()
+                  for x in (k, v))
+        want = oracle.coldstore_record(i + 1, i % 5, 100 * i, tokens, kv_heads, head_dim, 1, kp, vp)
+        got = bytes(frame[: HDR + 16 * tokens]) + kp + vp + bytes(frame[-FTR:])
+        assert got == want, (i, tokens, first)

@@ -18,18 +18,19 @@
 // record_payloads writes), so a stored record can be verified before any of
 // its bytes reach the pool.
 //
-// Two launches:
+// Three launches:
 //   * token_hashes_kernel: one lane per (record, K/V, token) computes the
 //     FNV-1a-64 of that token's bytes over all heads (cold_store.rs:725-742).
 //     These lanes are independent, so this launch streams the payloads at
 //     close to HBM rate;
-//   * frame_kernel: one lane of each of two wavefronts per record computes
-//     the payload and hash-table checksums (FNV-1a-64, cold_store.rs:909-922),
-//     assembles the header, then runs the record checksum and SHA-256
-//     (FIPS 180-4) over header | hashes | K | V and writes the footer.  FNV-1a
-//     and SHA-256 are sequential chains over the record's bytes, so this
-//     launch is bounded by the longest chain (SHA-256 of one record), not by
-//     bandwidth; it is meant for sealing or verifying many records at once.
+//   * payload_sums_kernel: the FNV-1a-64 checksums of the K and V payloads
+//     (cold_store.rs:909-922), one wavefront per payload;
+//   * frame_kernel: the hash-table checksums and the header, then the record
+//     checksum and SHA-256 (FIPS 180-4) over header | hashes | K | V and the
+//     footer, three wavefronts per 64 records.  SHA-256 is a sequential chain
+//     over the record's bytes, so this launch is bounded by the longest chain,
+//     not by bandwidth; it is meant for sealing or verifying many records at
+//     once.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -41,6 +42,7 @@ constexpr uint64_t kFnvOffset = 0xcbf29ce484222325ull;
 constexpr uint64_t kFnvPrime = 0x100000001b3ull;
 constexpr int kHeaderWords = kRecordHeaderBytes / 4;   // 26
 constexpr int kFooterWords = kRecordFooterBytes / 4;   // 14
+constexpr int kKeySumWord = 18;                        // K payload checksum, V's follows
 
 __device__ __forceinline__ uint64_t fnv_byte(uint64_t s, uint32_t b) { return (s ^ b) * kFnvPrime; }
 
@@ -175,6 +177,122 @@ __global__ __launch_bounds__(256) void token_hashes_kernel(FramesCodecLaunch a) 
     table[part * (int)r.tokens + token] = s;
 }
 
+// FNV-1a over the little-endian bytes of a payload by one wavefront, each lane
+// on a segment of up to 512 bytes of a 32 KiB tile.  One step is
+// s' = (s ^ b) P mod 2^64, and s ^ b = s + d with d set by b and the low byte of
+// s alone.  So once the low byte l at the start of a segment is known, the
+// segment maps any state s with that low byte to (s - l) P^n + C, where C is
+// the segment's own chain started from l, and the lanes' results combine in 64
+// multiply-adds.
+//
+// The low byte runs by itself: l' = (l ^ b) 0xb3 mod 256.  Bit j of it depends
+// on bits 0..j only, and flipping bit j of the start flips just bit j of the
+// end (0xb3 is odd).  So with bits 0..j-1 of every start known and bit j taken
+// as zero, the parity of the end bits of the segments before one is its true
+// bit j.  A pass runs the byte chain twice, packed in 16-bit halves, with bit
+// j zero and one, which settles bits j and j + 1.  Four such passes of three
+// cheap instructions per byte and one pass of the full chain, over segments
+// held in registers, replace one full chain over the whole payload.  For 2,016
+// records of two 32 KiB payloads: 0.6 ms as the first part of the frame
+// kernel's chain; 223 us with 32 lanes re-reading their segments for eight
+// passes; 94 us here.
+constexpr int kSumLanes = 64;
+constexpr int kSumChunks = 32;  // of a segment, in registers
+typedef unsigned short ushort2_t __attribute__((ext_vector_type(2)));
+
+constexpr uint64_t fnv_prime_power(int n) {
+    uint64_t p = 1;
+    for (int i = 0; i < n; ++i) p *= kFnvPrime;
+    return p;
+}
+
+__global__ __launch_bounds__(256) void payload_sums_kernel(FramesCodecLaunch a) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + threadIdx.x / 64));
+    const int lane = threadIdx.x & 63;
+    const int rec = wave / 2, part = wave % 2;  // one wavefront per (record, K or V)
+    if (rec >= a.count) return;
+    const RecordDesc r = a.records[rec];
+    if (!record_ok(a, r)) return;
+    const int tokens = (int)r.tokens;
+    const int row_bytes = a.head_dim * 2, row_chunks = row_bytes / 16;
+    const int chunks = a.kv_heads * tokens * row_chunks;  // of the payload
+    const PayloadAt at = payload_at(a, part ? a.v_pool : a.k_pool, r, rec, row_bytes);
+    const uint64_t below = ((uint64_t)1 << lane) - 1;
+
+    uint64_t sum = kFnvOffset;
+    for (int t0 = 0; t0 < chunks; t0 += kSumLanes * kSumChunks) {
+        const int here = min(chunks - t0, kSumLanes * kSumChunks);
+        const int per = (here + kSumLanes - 1) / kSumLanes;
+        const int c0 = min(lane * per, here), n = min(c0 + per, here) - c0;
+        // The segment: chunk t0 + c0 lies in row (t0 + c0) / row_chunks of the
+        // head-major rows.
+        const int row = (t0 + c0) / row_chunks, head = row / tokens;
+        ChunkWalk walk;
+        walk.head_base = at.base + (int64_t)head * at.head_stride;
+        walk.row = walk.head_base + (int64_t)(row - head * tokens) * row_bytes;
+        walk.head_stride = at.head_stride;
+        walk.row_bytes = row_bytes;
+        walk.col = (t0 + c0) % row_chunks * 16;
+        walk.rows_left = tokens - 1 - (row - head * tokens);
+        walk.rows_per_head = tokens;
+        u32x4_t c[kSumChunks];
+#pragma unroll
+        for (int i = 0; i < kSumChunks; ++i) {
+            if (i < n) {
+                c[i] = *walk.ptr();
+                walk.advance();
+            }
+        }
+        uint32_t start = 0;
+#pragma unroll 1
+        for (int j = 0; j < 8; j += 2) {
+            ushort2_t l = {(unsigned short)start, (unsigned short)(start | (1u << j))};
+            const ushort2_t prime = {(unsigned short)(kFnvPrime & 0xff), (unsigned short)(kFnvPrime & 0xff)};
+#pragma unroll
+            for (int i = 0; i < kSumChunks; ++i) {
+                if (i >= n) continue;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        // byte e of the word in both halves (0x0c: zero)
+                        const uint32_t b = __builtin_amdgcn_perm(0, c[i][k], 0x0c000c00u + 0x00010001u * e);
+                        l = (l ^ __builtin_bit_cast(ushort2_t, b)) * prime;
+                    }
+            }
+            auto settle = [&](uint32_t end, int bit) __attribute__((always_inline)) {
+                const uint64_t ends = __builtin_amdgcn_ballot_w64(((end >> bit) & 1u) != 0);
+                return ((uint32_t)(sum >> bit) ^ (uint32_t)__popcll(ends & below)) & 1u;
+            };
+            const uint32_t low = settle(l[0], j);
+            const uint32_t high = settle(low ? l[1] : l[0], j + 1);
+            start |= low << j | high << (j + 1);
+        }
+        uint64_t chain = start, power = 1;
+#pragma unroll
+        for (int i = 0; i < kSumChunks; ++i)
+            if (i < n) chain = fnv_chunk(chain, c[i]);
+        uint64_t square = fnv_prime_power(16);  // of one chunk
+        for (int e = n; e; e >>= 1, square *= square)
+            if (e & 1) power *= square;
+#pragma unroll 1
+        for (int i = 0; i < kSumLanes; ++i) {
+            auto of = [&](uint64_t x) __attribute__((always_inline)) {
+                return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)x, i) |
+                       ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), i) << 32);
+            };
+            sum = (sum - (uint32_t)__builtin_amdgcn_readlane((int)start, i)) * of(power) + of(chain);
+        }
+    }
+    // Left in the header words the checksums belong to; the frame kernel reads
+    // them there.
+    if (lane == 0) {
+        uint32_t *words = reinterpret_cast<uint32_t *>(static_cast<unsigned char *>(a.frames) + (int64_t)rec * a.frame_bytes);
+        words[kKeySumWord + 2 * part] = (uint32_t)sum;
+        words[kKeySumWord + 2 * part + 1] = (uint32_t)(sum >> 32);
+    }
+}
+
 // ---- SHA-256 (FIPS 180-4) -------------------------------------------------
 
 __device__ __constant__ uint32_t kSha256K[64] = {
@@ -188,150 +306,57 @@ __device__ __constant__ uint32_t kSha256K[64] = {
     0x748f82eeu, 0x78a5636fu, 0x84c87814u, 0x8cc70208u, 0x90befffau, 0xa4506cebu, 0xbef9a3f7u, 0xc67178f2u};
 
 __device__ __forceinline__ uint32_t rotr(uint32_t x, int n) { return (x >> n) | (x << (32 - n)); }
-
-// One compression of the 16 big-endian message words w into h.
-__device__ __forceinline__ void sha256_compress(uint32_t h[8], uint32_t w[16]) {
-    uint32_t a = h[0], b = h[1], c = h[2], d = h[3], e = h[4], f = h[5], g = h[6], k = h[7];
-#pragma unroll
-    for (int i = 0; i < 64; ++i) {
-        uint32_t wi;
-        if (i < 16) {
-            wi = w[i];
-        } else {
-            const uint32_t w15 = w[(i + 1) & 15], w2 = w[(i + 14) & 15];
-            const uint32_t s0 = rotr(w15, 7) ^ rotr(w15, 18) ^ (w15 >> 3);
-            const uint32_t s1 = rotr(w2, 17) ^ rotr(w2, 19) ^ (w2 >> 10);
-            wi = w[i & 15] + s0 + w[(i + 9) & 15] + s1;
-            w[i & 15] = wi;
-        }
-        const uint32_t t1 = k + (rotr(e, 6) ^ rotr(e, 11) ^ rotr(e, 25)) + ((e & f) ^ (~e & g)) + kSha256K[i] + wi;
-        const uint32_t t2 = (rotr(a, 2) ^ rotr(a, 13) ^ rotr(a, 22)) + ((a & b) ^ (a & c) ^ (b & c));
-        k = g;
-        g = f;
-        f = e;
-        e = d + t1;
-        d = c;
-        c = b;
-        b = a;
-        a = t1 + t2;
-    }
-    h[0] += a; h[1] += b; h[2] += c; h[3] += d;
-    h[4] += e; h[5] += f; h[6] += g; h[7] += k;
+// Three-input bit functions in one instruction each (v_bitop3_b32; the truth
+// table is the function of 0xf0, 0xcc and 0xaa).
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+}
+__device__ __forceinline__ uint32_t choose(uint32_t a, uint32_t b, uint32_t c) {  // a ? b : c
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0xca);
+}
+__device__ __forceinline__ uint32_t majority(uint32_t a, uint32_t b, uint32_t c) {
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0xe8);
 }
 
-// Streams `n` 16-byte chunks of a walk through `f`, keeping N loads in
-// flight ahead of the chain.  `group` runs after every N chunks (and once
-// after the tail), outside the unrolled body, so what it inlines appears
-// once.
-template <int N, class F, class G>
-__device__ __forceinline__ void stream_chunks(ChunkWalk ld, int64_t n, F &&f, G &&group) {
-    u32x4_t buf[N];
+// Sixteen message words (big-endian values) extended in place to the schedule
+// of rounds r .. r + 15, r a multiple of 16 above zero.
+__device__ __forceinline__ void sha256_extend(uint32_t w[16]) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-        if (i < n) {
-            buf[i] = *ld.ptr();
-            ld.advance();
-        }
+    for (int i = 0; i < 16; ++i) {
+        const uint32_t w15 = w[(i + 1) & 15], w2 = w[(i + 14) & 15];
+        const uint32_t s0 = xor3(rotr(w15, 7), rotr(w15, 18), w15 >> 3);
+        const uint32_t s1 = xor3(rotr(w2, 17), rotr(w2, 19), w2 >> 10);
+        w[i] += s0 + w[(i + 9) & 15] + s1;
     }
-    int64_t c = 0;
-    for (; c + N <= n; c += N) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const u32x4_t cur = buf[i];
-            if (c + N + i < n) {
-                buf[i] = *ld.ptr();
-                ld.advance();
-            }
-            f(cur);
-        }
-        group();
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-        if (c + i < n) f(buf[i]);
-    group();
 }
-
-// The same over two walks of equal length, in lockstep.
-template <int N, class F>
-__device__ __forceinline__ void stream_chunks2(ChunkWalk la, ChunkWalk lb, int64_t n, F &&f) {
-    u32x4_t ba[N], bb[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        if (i < n) {
-            ba[i] = *la.ptr();
-            bb[i] = *lb.ptr();
-            la.advance();
-            lb.advance();
-        }
-    }
-    int64_t c = 0;
-    for (; c + N <= n; c += N) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const u32x4_t ca = ba[i], cb = bb[i];
-            if (c + N + i < n) {
-                ba[i] = *la.ptr();
-                bb[i] = *lb.ptr();
-                la.advance();
-                lb.advance();
-            }
-            f(ca, cb);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-        if (c + i < n) f(ba[i], bb[i]);
-}
-
-// SHA-256 message state of one lane.  Words enter a 64-word ring in LDS
-// (which takes a dynamic index); `drain` compresses every complete block.
-constexpr int kFrameThreads = 64;
-constexpr int kRingWords = 64;
-
-struct ShaStream {
-    uint32_t *ring;  // LDS, kRingWords words at stride kFrameThreads
-    uint32_t h[8];
-    uint32_t wpos, rpos;
-
-    __device__ __forceinline__ void init(uint32_t *lds) {
-        ring = lds;
-        h[0] = 0x6a09e667u; h[1] = 0xbb67ae85u; h[2] = 0x3c6ef372u; h[3] = 0xa54ff53au;
-        h[4] = 0x510e527fu; h[5] = 0x9b05688cu; h[6] = 0x1f83d9abu; h[7] = 0x5be0cd19u;
-        wpos = rpos = 0;
-    }
-    __device__ __forceinline__ void push_be(uint32_t be) {
-        ring[(wpos & (kRingWords - 1)) * kFrameThreads] = be;
-        ++wpos;
-    }
-    __device__ __forceinline__ void drain() {
-        while (wpos - rpos >= 16) {
-            uint32_t w[16];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) w[i] = ring[((rpos + i) & (kRingWords - 1)) * kFrameThreads];
-            sha256_compress(h, w);
-            rpos += 16;
-        }
-    }
-};
 
 __device__ __forceinline__ uint32_t lo32(uint64_t x) { return (uint32_t)x; }
 __device__ __forceinline__ uint32_t hi32(uint64_t x) { return (uint32_t)(x >> 32); }
 
-constexpr int kFramePrefetch = 8;
+// Three wavefronts per 64 records, lane = record, in step over the 64-byte
+// blocks of header | tables | K | V | padding:
+//   * the schedule wavefront loads block i + 2, extends it to its 64 round
+//     words and leaves them, constants added, in LDS (and the sixteen message
+//     words as they lie in the record);
+//   * the rounds wavefront runs the 64 rounds of block i;
+//   * the checksum wavefront runs the record's FNV-1a over block i.
+// A lane's instructions issue every four clocks whatever its neighbours do, so
+// the chain is as long as its instruction count: the rounds alone are 14
+// instructions each, and everything else of SHA-256 (8 to 10 more, the loads
+// and byte swaps) runs on another SIMD.  2,016 records of 64 KiB payloads:
+// 4.41 ms with the schedule, the message ring and the payload checksums on
+// the rounds' wavefront, 2.11 ms here (1,030 blocks of 64 rounds).
+constexpr int kFrameThreads = 64;  // records per workgroup
+constexpr int kFrameRoles = 3;
+enum { kRounds = 0, kSchedule = 1, kChecksum = 2 };
 
-// Two wavefronts per 64 records, each running one chain per lane: in the
-// first pass wavefront 0 checksums the K payloads and wavefront 1 the V
-// payloads; in the second, over header | tables | K | V, wavefront 0 runs
-// SHA-256 and wavefront 1 the record FNV.  A lane's chains are sequential,
-// so splitting them over the two wavefronts (on different SIMDs) shortens
-// the critical path; they meet through LDS at two barriers.
-__global__ __launch_bounds__(2 * kFrameThreads) void frame_kernel(FramesCodecLaunch a) {
-    __shared__ uint32_t rings[kRingWords * kFrameThreads];
-    __shared__ uint64_t payload_sums[2][kFrameThreads];
-    __shared__ uint64_t record_sums[kFrameThreads];
+__global__ __launch_bounds__(kFrameRoles * kFrameThreads) void frame_kernel(FramesCodecLaunch a) {
+    // [block % 4][four words][lane]
+    __shared__ u32x4_t rounds_lds[4][16][kFrameThreads];
+    __shared__ u32x4_t message_lds[4][4][kFrameThreads];
+    __shared__ uint64_t sums[kFrameRoles][kFrameThreads];
     const int lane = threadIdx.x & (kFrameThreads - 1);
-    const int role = threadIdx.x / kFrameThreads;  // wavefront 0 or 1
+    const int role = __builtin_amdgcn_readfirstlane(threadIdx.x / kFrameThreads);
     const int rec = blockIdx.x * kFrameThreads + lane;
     const bool live = rec < a.count;
     RecordDesc r = {};
@@ -341,142 +366,240 @@ __global__ __launch_bounds__(2 * kFrameThreads) void frame_kernel(FramesCodecLau
                                                          (int64_t)(live ? rec : 0) * a.frame_bytes);
     const int frame_words_n = (int)(a.frame_bytes / 4);
     const int tokens = valid ? (int)r.tokens : 0;
-    const int row_bytes = a.head_dim * 2;
+    const int row_bytes = a.head_dim * 2, row_chunks = row_bytes / 16;
     const int64_t payload_len = (int64_t)a.kv_heads * tokens * row_bytes;
-    const int64_t payload_chunks = payload_len / 16;
     RecordDesc rv = r;
     if (!valid) rv = RecordDesc{0, 0, 0, 1, 0, 0};
     const PayloadAt kat = payload_at(a, a.k_pool, rv, valid ? rec : 0, row_bytes);
     const PayloadAt vat = payload_at(a, a.v_pool, rv, valid ? rec : 0, row_bytes);
-    const unsigned char *kpage = kat.base;
-    const unsigned char *vpage = vat.base;
-
-    // Head-major payload of `tokens` rows per head.
-    auto payload_walk = [&](const unsigned char *page) __attribute__((always_inline)) {
-        ChunkWalk w;
-        w.head_base = page;
-        w.row = page;
-        w.head_stride = kat.head_stride;
-        w.row_bytes = row_bytes;
-        w.col = 0;
-        w.rows_left = tokens - 1;
-        w.rows_per_head = tokens;
-        return w;
-    };
-    auto no_group = []() __attribute__((always_inline)) {};
-
-    // Pass 1: payload checksums, K on wavefront 0 and V on wavefront 1.
-    {
-        uint64_t sum = kFnvOffset;
-        if (valid)
-            stream_chunks<kFramePrefetch>(payload_walk(role == 0 ? kpage : vpage), payload_chunks,
-                                          [&](const u32x4_t &c) __attribute__((always_inline)) {
-                                              sum = fnv_chunk(sum, c);
-                                          },
-                                          no_group);
-        payload_sums[role][lane] = sum;
-    }
-    __syncthreads();
-    const uint64_t key_sum = payload_sums[0][lane], value_sum = payload_sums[1][lane];
 
     // Hash-table checksums over the little-endian u64 tables (written by
-    // token_hashes_kernel into this frame) and the header
-    // (cold_store.rs:291-309), on both wavefronts.
+    // token_hashes_kernel into this frame): K's on one wavefront, V's on
+    // another.
     const uint32_t *tables = frame_words + kHeaderWords;
-    uint64_t key_hashes_sum = kFnvOffset, value_hashes_sum = kFnvOffset;
-    for (int i = 0; i < 2 * tokens; ++i) key_hashes_sum = fnv_word(key_hashes_sum, tables[i]);
-    for (int i = 2 * tokens; i < 4 * tokens; ++i) value_hashes_sum = fnv_word(value_hashes_sum, tables[i]);
-    uint32_t hdr[kHeaderWords];
-    hdr[0] = 0x564b5354u;  // "TSKV"
-    hdr[1] = 0x34304750u;  // "PG04"
-    hdr[2] = kRecordVersion;
-    hdr[3] = kRecordHeaderBytes;
-    hdr[4] = lo32(r.page_id);
-    hdr[5] = hi32(r.page_id);
-    hdr[6] = r.layer;
-    hdr[7] = 0u;
-    hdr[8] = lo32(r.token_start);
-    hdr[9] = hi32(r.token_start);
-    hdr[10] = r.tokens;
-    hdr[11] = (uint32_t)a.kv_heads;
-    hdr[12] = (uint32_t)a.head_dim;
-    hdr[13] = a.tile;
-    hdr[14] = lo32((uint64_t)payload_len);
-    hdr[15] = hi32((uint64_t)payload_len);
-    hdr[16] = lo32((uint64_t)payload_len);
-    hdr[17] = hi32((uint64_t)payload_len);
-    hdr[18] = lo32(key_sum);
-    hdr[19] = hi32(key_sum);
-    hdr[20] = lo32(value_sum);
-    hdr[21] = hi32(value_sum);
-    hdr[22] = lo32(key_hashes_sum);
-    hdr[23] = hi32(key_hashes_sum);
-    hdr[24] = lo32(value_hashes_sum);
-    hdr[25] = hi32(value_hashes_sum);
-
-    // Pass 2 over header | tables | K | V: SHA-256 on wavefront 0, the record
-    // FNV on wavefront 1.
-    const uint64_t record_len =
-        (uint64_t)kRecordHeaderBytes + 16ull * tokens + 2ull * (uint64_t)payload_len + kRecordFooterBytes;
-    ShaStream sha;
-    sha.init(rings + lane);
-    if (role == 0) {
-        if (valid) {
+    if (role != kChecksum) {
+        uint64_t sum = kFnvOffset;
+        const uint2 *t = reinterpret_cast<const uint2 *>(tables) + role * tokens;
+        constexpr int kAhead = 8;
+        for (int i0 = 0; i0 < tokens; i0 += kAhead) {
+            uint2 h[kAhead];
 #pragma unroll
-            for (int i = 0; i < kHeaderWords; ++i) sha.push_be(__builtin_bswap32(hdr[i]));
-            sha.drain();
-            for (int i = 0; i < 4 * tokens; ++i) {
-                sha.push_be(__builtin_bswap32(tables[i]));
-                if (sha.wpos - sha.rpos >= 16) sha.drain();
-            }
-            auto push_chunk = [&](const u32x4_t &c) __attribute__((always_inline)) {
-                sha.push_be(__builtin_bswap32(c[0]));
-                sha.push_be(__builtin_bswap32(c[1]));
-                sha.push_be(__builtin_bswap32(c[2]));
-                sha.push_be(__builtin_bswap32(c[3]));
-            };
-            auto drain = [&]() __attribute__((always_inline)) { sha.drain(); };
-            stream_chunks<kFramePrefetch>(payload_walk(kpage), payload_chunks, push_chunk, drain);
-            stream_chunks<kFramePrefetch>(payload_walk(vpage), payload_chunks, push_chunk, drain);
-            // FIPS 180-4 padding: 0x80, zeros to 56 mod 64, 64-bit big-endian length.
-            const uint64_t message_bits = (record_len - kRecordFooterBytes) * 8;
-            sha.push_be(0x80000000u);
-            while (((sha.wpos - sha.rpos) & 15) != 14) sha.push_be(0u);
-            sha.push_be(hi32(message_bits));
-            sha.push_be(lo32(message_bits));
-            sha.drain();
-        }
-    } else {
-        uint64_t record_sum = kFnvOffset;
-        if (valid) {
+            for (int i = 0; i < kAhead; ++i) h[i] = t[min(i0 + i, tokens - 1)];
 #pragma unroll
-            for (int i = 0; i < kHeaderWords; ++i) record_sum = fnv_word(record_sum, hdr[i]);
-            for (int i = 0; i < 4 * tokens; ++i) record_sum = fnv_word(record_sum, tables[i]);
-            auto fnv_of = [&](const u32x4_t &c) __attribute__((always_inline)) { record_sum = fnv_chunk(record_sum, c); };
-            stream_chunks<kFramePrefetch>(payload_walk(kpage), payload_chunks, fnv_of, no_group);
-            stream_chunks<kFramePrefetch>(payload_walk(vpage), payload_chunks, fnv_of, no_group);
+            for (int i = 0; i < kAhead; ++i)
+                if (i0 + i < tokens) sum = fnv_word(fnv_word(sum, h[i].x), h[i].y);
         }
-        record_sums[lane] = record_sum;
+        sums[role][lane] = sum;
     }
     __syncthreads();
-    if (role != 0 || !live) return;
-    if (!valid) {
-        for (int i = 0; i < frame_words_n; ++i) frame_words[i] = 0u;
-        return;
+    const uint64_t record_len =
+        (uint64_t)kRecordHeaderBytes + 16ull * tokens + 2ull * (uint64_t)payload_len + kRecordFooterBytes;
+    // The header (cold_store.rs:291-309); the payload checksums already lie in
+    // it (payload_sums_kernel).
+    if (role == kRounds && valid) {
+        const uint64_t key_hashes_sum = sums[0][lane], value_hashes_sum = sums[1][lane];
+        frame_words[0] = 0x564b5354u;  // "TSKV"
+        frame_words[1] = 0x34304750u;  // "PG04"
+        frame_words[2] = kRecordVersion;
+        frame_words[3] = kRecordHeaderBytes;
+        frame_words[4] = lo32(r.page_id);
+        frame_words[5] = hi32(r.page_id);
+        frame_words[6] = r.layer;
+        frame_words[7] = 0u;
+        frame_words[8] = lo32(r.token_start);
+        frame_words[9] = hi32(r.token_start);
+        frame_words[10] = r.tokens;
+        frame_words[11] = (uint32_t)a.kv_heads;
+        frame_words[12] = (uint32_t)a.head_dim;
+        frame_words[13] = a.tile;
+        frame_words[14] = lo32((uint64_t)payload_len);
+        frame_words[15] = hi32((uint64_t)payload_len);
+        frame_words[16] = lo32((uint64_t)payload_len);
+        frame_words[17] = hi32((uint64_t)payload_len);
+        frame_words[22] = lo32(key_hashes_sum);
+        frame_words[23] = hi32(key_hashes_sum);
+        frame_words[24] = lo32(value_hashes_sum);
+        frame_words[25] = hi32(value_hashes_sum);
+        for (int i = kHeaderWords + 4 * tokens; i < frame_words_n - kFooterWords; ++i) frame_words[i] = 0u;
     }
-    const uint64_t record_sum = record_sums[lane];
+    __syncthreads();  // the header is read back as message words below
+
+    // The message: head words (header and tables, as they lie in the frame),
+    // payload words (K then V, whole 16-byte chunks), the 0x80 byte, zeros and
+    // the bit length.  The payload starts at word 2 of a group of four.
+    const int head_words = kHeaderWords + 4 * tokens;
+    const int part_chunks = (int)(payload_len / 16);
+    const int payload_words = 8 * part_chunks;
+    const int message_words = head_words + payload_words;
+    const int blocks = valid ? (message_words + 3 + 15) / 16 : 0;
+    int most = blocks;
 #pragma unroll
-    for (int i = 0; i < kHeaderWords; ++i) frame_words[i] = hdr[i];
-    for (int i = kHeaderWords + 4 * tokens; i < frame_words_n - kFooterWords; ++i) frame_words[i] = 0u;
-    uint32_t *footer = frame_words + frame_words_n - kFooterWords;
-    footer[0] = 0x564b5354u;  // "TSKV"
-    footer[1] = 0x54494d43u;  // "CMIT"
-    footer[2] = lo32(record_sum);
-    footer[3] = hi32(record_sum);
-    footer[4] = lo32(record_len);
-    footer[5] = hi32(record_len);
+    for (int m = 32; m >= 1; m >>= 1) most = max(most, __shfl_xor(most, m, 64));
+    most = __builtin_amdgcn_readfirstlane(most);
+
+    // Where chunk i of K then V lies.  A payload whose heads follow each other
+    // without a gap (a whole page, or staging) is one run.
+    const bool run = kat.head_stride == (int64_t)tokens * row_bytes;
+    auto chunk_at = [&](int i) __attribute__((always_inline)) {
+        const bool v = i >= part_chunks;
+        const int c = v ? i - part_chunks : i;
+        const unsigned char *base = v ? vat.base : kat.base;
+        if (run) return base + (int64_t)c * 16;
+        const int row = c / row_chunks, head = row / tokens;
+        return base + head * kat.head_stride + (int64_t)(row - head * tokens) * row_bytes + (c - row * row_chunks) * 16;
+    };
+
+    if (role == kSchedule) {
+        // Block b is inside the payload for most of a record: its words are
+        // the last two of chunk c, chunks c + 1 .. c + 3 and the first two of
+        // chunk c + 4.
+        auto inside = [&](int b) __attribute__((always_inline)) {
+            const int o = b * 16 - head_words;
+            return o >= 2 && o + 16 <= payload_words;
+        };
+        constexpr int kAhead = 2;  // blocks in flight
+        u32x4_t ahead[kAhead][5];
+        auto fetch = [&](u32x4_t (&c)[5], int b) __attribute__((always_inline)) {
+            if (!inside(b)) return;
+            const int c0 = (b * 16 - head_words - 2) / 4;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) footer[6 + i] = __builtin_bswap32(sha.h[i]);
+            for (int k = 0; k < 5; ++k) c[k] = *reinterpret_cast<const u32x4_t *>(chunk_at(c0 + k));
+        };
+        auto produce = [&](const u32x4_t (&c)[5], int b) __attribute__((always_inline)) {
+            uint32_t w[16];
+            if (inside(b)) {
+                w[0] = c[0][2];
+                w[1] = c[0][3];
+#pragma unroll
+                for (int k = 0; k < 12; ++k) w[2 + k] = c[1 + k / 4][k % 4];
+                w[14] = c[4][0];
+                w[15] = c[4][1];
+            } else {
+                const uint64_t bits = (record_len - kRecordFooterBytes) * 8;
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    const int g = b * 16 + j, o = g - head_words;
+                    uint32_t x = 0;
+                    if (b < blocks) {
+                        if (g < head_words) x = frame_words[g];
+                        else if (o < payload_words) x = reinterpret_cast<const uint32_t *>(chunk_at(o / 4))[o % 4];
+                        else if (g == message_words) x = 0x80u;
+                        else if (g == blocks * 16 - 2) x = __builtin_bswap32(hi32(bits));
+                        else if (g == blocks * 16 - 1) x = __builtin_bswap32(lo32(bits));
+                    }
+                    w[j] = x;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                message_lds[b & 3][k][lane] = u32x4_t{w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]};
+#pragma unroll
+            for (int j = 0; j < 16; ++j) w[j] = __builtin_bswap32(w[j]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (q) sha256_extend(w);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    u32x4_t x;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[e] = w[4 * k + e] + kSha256K[16 * q + 4 * k + e];
+                    rounds_lds[b & 3][4 * q + k][lane] = x;
+                }
+            }
+        };
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) fetch(ahead[k], k);
+        produce(ahead[0], 0);
+        fetch(ahead[0], kAhead);
+        for (int b = 0; b < most; b += kAhead) {
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                if (b + k >= most) break;
+                const int next = (k + 1) % kAhead;
+                produce(ahead[next], b + k + 1);
+                fetch(ahead[next], b + k + 1 + kAhead);
+                __syncthreads();
+            }
+        }
+    } else if (role == kRounds) {
+        uint32_t h[8] = {0x6a09e667u, 0xbb67ae85u, 0x3c6ef372u, 0xa54ff53au,
+                         0x510e527fu, 0x9b05688cu, 0x1f83d9abu, 0x5be0cd19u};
+        // Barrier b: blocks up to b + 1 are in LDS, and the place of block
+        // b - 2 is free.  The first words of block b + 1 are read ahead of
+        // the last rounds of block b.
+        constexpr int kFirst = 4;
+        u32x4_t first[kFirst] = {};
+        for (int b = 0; b < most; ++b) {
+            __syncthreads();
+            if (b >= blocks) continue;
+            if (b == 0) {
+#pragma unroll
+                for (int k = 0; k < kFirst; ++k) first[k] = rounds_lds[0][k][lane];
+            }
+            uint32_t s[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s[i] = h[i];
+#pragma unroll
+            for (int i = 0; i < 64; i += 4) {
+                const u32x4_t kw = i / 4 < kFirst ? first[i / 4 % kFirst] : rounds_lds[b & 3][i / 4][lane];
+                if (i == 4 * kFirst) {
+#pragma unroll
+                    for (int k = 0; k < kFirst; ++k) first[k] = rounds_lds[(b + 1) & 3][k][lane];
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    // s[(0 - i - e) & 7] is the round's a, and so on: the
+                    // state turns instead of moving
+                    const int n = (i + e) & 7;
+                    const uint32_t A = s[(8 - n) & 7], B = s[(9 - n) & 7], C = s[(10 - n) & 7];
+                    const uint32_t E = s[(12 - n) & 7], F = s[(13 - n) & 7], G = s[(14 - n) & 7];
+                    const uint32_t t1 = s[(15 - n) & 7] + kw[e] + xor3(rotr(E, 6), rotr(E, 11), rotr(E, 25)) +
+                                        choose(E, F, G);
+                    s[(11 - n) & 7] += t1;
+                    s[(15 - n) & 7] = t1 + xor3(rotr(A, 2), rotr(A, 13), rotr(A, 22)) + majority(A, B, C);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) h[i] += s[i];
+        }
+        __syncthreads();  // the checksum wavefront is done
+        if (!live) return;
+        if (!valid) {
+            for (int i = 0; i < frame_words_n; ++i) frame_words[i] = 0u;
+            return;
+        }
+        const uint64_t record_sum = sums[kChecksum][lane];
+        uint32_t *footer = frame_words + frame_words_n - kFooterWords;
+        footer[0] = 0x564b5354u;  // "TSKV"
+        footer[1] = 0x54494d43u;  // "CMIT"
+        footer[2] = lo32(record_sum);
+        footer[3] = hi32(record_sum);
+        footer[4] = lo32(record_len);
+        footer[5] = hi32(record_len);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) footer[6 + i] = __builtin_bswap32(h[i]);
+        return;
+    } else {
+        uint64_t record_sum = kFnvOffset;
+        for (int b = 0; b < most; ++b) {
+            __syncthreads();
+            const int n = message_words - b * 16;  // message words left
+            if (!valid || n <= 0) continue;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const u32x4_t c = message_lds[b & 3][k][lane];
+                if (n >= 16) {
+                    record_sum = fnv_chunk(record_sum, c);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (4 * k + e < n) record_sum = fnv_word(record_sum, c[e]);
+                }
+            }
+        }
+        sums[kChecksum][lane] = record_sum;
+    }
+    __syncthreads();
 }
 
 // Payload moves between pool pages and contiguous staging: staging slot i
@@ -525,8 +648,11 @@ hipError_t launch_record_frames(const FramesCodecLaunch &a, hipStream_t stream) 
     const int64_t lanes = (int64_t)a.count * 2 * a.page_tokens;
     hipLaunchKernelGGL(token_hashes_kernel, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, stream, a);
     if (hipError_t e = hipGetLastError()) return e;
+    const int64_t sum_lanes = (int64_t)a.count * 2 * kSumLanes;
+    hipLaunchKernelGGL(payload_sums_kernel, dim3((unsigned)((sum_lanes + 255) / 256)), dim3(256), 0, stream, a);
+    if (hipError_t e = hipGetLastError()) return e;
     hipLaunchKernelGGL(frame_kernel, dim3((unsigned)((a.count + kFrameThreads - 1) / kFrameThreads)),
-                       dim3(2 * kFrameThreads), 0, stream, a);
+                       dim3(kFrameRoles * kFrameThreads), 0, stream, a);
     return hipGetLastError();
 }
 
