@@ -172,6 +172,7 @@ private:
     void injected_error(int layer);
     void check_healthy(int seq) const;
     void *alloc(size_t bytes);
+    void release();
     void chunk(int seq, const int32_t *ids, int n, int64_t prior);
     // The page pool of every layer (one allocation each for K and V) and the
     // pool pages of slot `seq` per layer, for the ColdStore device paths.
@@ -205,7 +206,9 @@ private:
     const int32_t *cancel_ = nullptr;
     std::vector<char> poisoned_;
     int inject_kind_ = 0, inject_layer_ = -1;
-    int32_t *table_ = nullptr, *ids_ = nullptr, *pos_ = nullptr, *next_ = nullptr;
+    int32_t *table_ = nullptr, *pos_ = nullptr, *row_ids_ = nullptr;
+    // one page-locked buffer: prompt or step ids, step positions, greedy tokens
+    int32_t *io_ = nullptr, *ids_ = nullptr, *host_pos_ = nullptr, *next_ = nullptr;
     uint16_t *x_ = nullptr, *q_ = nullptr, *k_ = nullptr, *v_ = nullptr, *qr_ = nullptr,
              *kr_ = nullptr, *attn_ = nullptr, *act_ = nullptr,
              *kd_ = nullptr, *vd_ = nullptr, *logits_ = nullptr;
