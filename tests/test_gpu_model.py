@@ -85,6 +85,25 @@ def test_argmax_bit_exact(ctx, rows, vocab):
     assert np.array_equal(out.cpu().numpy(), oracle.argmax_bf16(x, rows, vocab))
 
 
+@pytest.mark.parametrize("vocab", [8, 16, 8192, 8200, 131072, 131080, 140000, 8193])
+def test_argmax_equal_values_over_chunks_and_lanes(ctx, vocab):
+    # A lane takes 8 logits a load, the workgroup 8,192, a full batch of loads
+    # 131,072: few distinct values, so that the first of many equal ones has to
+    # win within a chunk, a lane, a wavefront and across them.  Exact.
+    rng = np.random.default_rng(vocab)
+    kinds = np.array([0.0, -0.0, -1.0, np.nan, -np.inf, -3.0], np.float32)
+    rows = [rng.choice(kinds[a:], vocab) for a in (0, 1, 2, 3, 5)]
+    last = rng.choice(kinds, vocab)
+    last[-1] = 1.0
+    pair = rng.choice(kinds[2:], vocab)
+    pair[rng.integers(0, vocab, 5)] = np.inf
+    x = oracle.write_bf16(np.stack(rows + [last, pair]).astype(np.float32).reshape(-1)).reshape(-1, vocab)
+    out = _dev_i32(np.full(len(x), -1))
+    ctx.argmax(to_torch(x), len(x), vocab, out)
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy(), oracle.argmax_bf16(x, len(x), vocab))
+
+
 def test_argmax_ties_nan_and_infinities(ctx):
     f = np.float32
     vocab = 600

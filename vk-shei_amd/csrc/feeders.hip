@@ -414,15 +414,23 @@ __global__ __launch_bounds__(256) void embed_kernel(const uint16_t *table, const
 }
 
 // Greedy token of each row of BF16 logits (llm_argmax, gpu_llm.cl:239-270),
-// one workgroup of 1024 lanes per row.  Every lane starts from (-inf, index 0)
-// and takes a value that is greater, or equal with a lower index: NaN never
+// one workgroup of 1024 lanes per row.  The rule: start from (-inf, index 0)
+// and take a value that is greater, or equal with a lower index, so NaN never
 // wins, the first index wins ties, and a row with nothing above -inf gives 0.
 // That rule makes the result independent of how elements are split over
-// lanes, so VEC lanes read 8 logits per 16-byte load (rows 16-byte aligned,
-// vocab % 8 == 0), four loads in flight.
+// lanes.  A lane visits its elements in rising order, where "greater" alone
+// decides.
+//
+// Bound by the lanes' comparisons, not by the row's bytes: one CU holds the
+// row.  VEC lanes (rows 16-byte aligned, vocab % 8 == 0) read 8 logits per
+// load with 16 loads in flight, which is a whole row of 131,072, keep only
+// the largest of the 8 and the chunk it came from (a comparison and a select
+// per logit, where tracking the index of each took eight instructions), and
+// one lane finds the logit in the winning chunk at the end.  A row of 128,256
+// logits: 13.2 us before, 6.8 us now; 20 rows 13.5 and 7.2.
 constexpr int kArgmaxThreads = 1024;
 
-__device__ __forceinline__ void argmax_take(float x, int i, float &best, int &index) {
+__device__ __forceinline__ void argmax_merge(float x, int i, float &best, int &index) {
     if (x > best || (x == best && i < index)) {
         best = x;
         index = i;
@@ -432,54 +440,75 @@ __device__ __forceinline__ void argmax_take(float x, int i, float &best, int &in
 template <bool VEC>
 __global__ __launch_bounds__(kArgmaxThreads) void argmax_kernel(const uint16_t *logits, int rows, int vocab,
                                                                 int32_t *out) {
-    __shared__ float values[kArgmaxThreads];
-    __shared__ int indices[kArgmaxThreads];
+    __shared__ float values[kArgmaxThreads / 64];
+    __shared__ int indices[kArgmaxThreads / 64];
     const int row = blockIdx.x;
     const int tid = threadIdx.x;
     const uint16_t *l = logits + (int64_t)row * vocab;
+    const uint4 *l4 = reinterpret_cast<const uint4 *>(l);
     float best = -INFINITY;
-    int index = 0;
+    int index = 0;  // VEC: of the chunk of 8
     if (VEC) {
-        const uint4 *l4 = reinterpret_cast<const uint4 *>(l);
         const int chunks = vocab / 8;
-        constexpr int U = 4;
+        constexpr int U = 16;
         for (int base = tid; base < chunks; base += kArgmaxThreads * U) {
             uint4 v[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int c = base + u * kArgmaxThreads;
-                if (c < chunks) v[u] = l4[c];
+                v[u] = l4[c < chunks ? c : base];
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int c = base + u * kArgmaxThreads;
-                if (c >= chunks) break;
                 const uint32_t words[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+                float m = -INFINITY;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    argmax_take(read_bf16((uint16_t)(words[k] & 0xffffu)), c * 8 + 2 * k, best, index);
-                    argmax_take(read_bf16((uint16_t)(words[k] >> 16)), c * 8 + 2 * k + 1, best, index);
+                    const float lo = __uint_as_float(words[k] << 16), hi = __uint_as_float(words[k] & 0xffff0000u);
+                    m = lo > m ? lo : m;
+                    m = hi > m ? hi : m;
+                }
+                // past the end the lane read its first chunk again: not greater
+                if (m > best) {
+                    best = m;
+                    index = base + u * kArgmaxThreads;
                 }
             }
         }
     } else {
-        for (int i = tid; i < vocab; i += kArgmaxThreads) argmax_take(read_bf16(l[i]), i, best, index);
-    }
-    values[tid] = best;
-    indices[tid] = index;
-    __syncthreads();
-    for (int stride = kArgmaxThreads / 2; stride > 0; stride >>= 1) {
-        if (tid < stride) {
-            const float ov = values[tid + stride];
-            const int oi = indices[tid + stride];
-            if (ov > values[tid] || (ov == values[tid] && oi < indices[tid])) {
-                values[tid] = ov;
-                indices[tid] = oi;
+        for (int i = tid; i < vocab; i += kArgmaxThreads) {
+            const float x = read_bf16(l[i]);
+            if (x > best) {
+                best = x;
+                index = i;
             }
         }
-        __syncthreads();
     }
-    if (tid == 0) out[row] = indices[0];
+#pragma unroll
+    for (int stride = 32; stride > 0; stride >>= 1)
+        argmax_merge(__shfl_xor(best, stride), __shfl_xor(index, stride), best, index);
+    if (tid % 64 == 0) {
+        values[tid / 64] = best;
+        indices[tid / 64] = index;
+    }
+    __syncthreads();
+    if (tid != 0) return;
+#pragma unroll
+    for (int w = 1; w < kArgmaxThreads / 64; ++w) argmax_merge(values[w], indices[w], best, index);
+    if (VEC) {
+        const uint4 v = l4[index];
+        const uint32_t words[4] = {v.x, v.y, v.z, v.w};
+        int at = 0;
+        if (best > -INFINITY) {
+#pragma unroll
+            for (int k = 7; k >= 0; --k) {
+                const float x = __uint_as_float(k % 2 ? words[k / 2] & 0xffff0000u : words[k / 2] << 16);
+                if (x == best) at = index * 8 + k;
+            }
+        }
+        index = at;
+    }
+    out[row] = index;
 }
 
 }  // namespace
