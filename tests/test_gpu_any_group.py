@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 import torch
 
+import mslim_attn
 import oracle
 from _data import from_torch, normal_bf16, to_torch
 
@@ -117,3 +118,36 @@ def _check_prefill(ctx, rng, qb, kb, vb, queries, prior, qh, kvh, d):
         ref = oracle.cpu_reference_decode(oracle.read_bf16(qb[r]), kb[:n], vb[:n], 1, qh, kvh, d)[1]
         for name, got in zip(("split", "unsplit", "unaligned"), outs):
             _check(got[r], ref, vb[:n], f"{name} row {r}")
+
+
+def test_prefill_first_call_under_capture():
+    # A shape that splits when run eagerly: a new context has no memory for the
+    # partials and can allocate none during capture, so it runs unsplit there.
+    queries, prior, qh, kvh, d = 600, 1500, 14, 2, 128
+    assert mslim_attn.prefill_split_tiles(queries, prior, qh, kvh, d) > 0
+    rng = np.random.default_rng(11)
+    q, k, v = (to_torch(normal_bf16(rng, s)) for s in ((queries, qh, d), (queries + prior, kvh, d),
+                                                       (queries + prior, kvh, d)))
+    got, want = torch.zeros_like(q), torch.zeros_like(q)
+    fresh = mslim_attn.Context()
+    try:
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        graph = torch.cuda.CUDAGraph()
+        fresh.set_stream(stream.cuda_stream)
+        with torch.cuda.graph(graph, stream=stream):
+            fresh.prefill_causal(q, k, v, got, queries, prior, qh, kvh, d)
+        fresh.use_torch_stream()
+        fresh.set_prefill_split(False)
+        fresh.prefill_causal(q, k, v, want, queries, prior, qh, kvh, d)
+        torch.cuda.synchronize()
+        for _ in range(3):
+            got.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, want)
+            fresh.prefill_causal(q, k, v, want, queries, prior, qh, kvh, d)
+        torch.cuda.synchronize()
+        del graph
+    finally:
+        fresh.close()

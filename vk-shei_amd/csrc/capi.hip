@@ -196,6 +196,10 @@ void decode_place_partials(mslim::DecodeLaunch &l, void *base) {
     l.partial_acc = reinterpret_cast<float *>(static_cast<char *>(base) + ml_bytes);
 }
 
+// Counters a new context holds of each kind (32 kv heads of the decode's 64
+// sequences; a portable decode splits only with 128 counters or fewer).
+constexpr int kFirstCounters = 2048;
+
 // At least n split counters in the context.  The kernels leave them at zero,
 // so they are cleared only when the buffer is (re)allocated or a launch failed.
 int split_counters(Context &c, size_t n) {
@@ -348,6 +352,23 @@ void *mslim_attn_ctx_new(void) {
         return nullptr;
     }
     c->proj_partial_bytes = mslim::kProjPartialBytes;
+    // Counters of fused merges and of pooled prefill, zero from here on: the
+    // portable decode never needs more, nor does a prefill that runs unsplit,
+    // so their first call may be under capture too.
+    void *counters = nullptr;
+    if (check_hip(hipMalloc(&counters, kFirstCounters * sizeof(int)), "hipMalloc split counters") ||
+        check_hip(hipMalloc(&c->prefill_counters, kFirstCounters * sizeof(int)), "hipMalloc prefill counters") ||
+        check_hip(mslim::launch_zero_i32(static_cast<int *>(counters), kFirstCounters, c->own_stream),
+                  "clear split counters") ||
+        check_hip(mslim::launch_zero_i32(static_cast<int *>(c->prefill_counters), kFirstCounters, c->own_stream),
+                  "clear prefill counters") ||
+        check_hip(hipStreamSynchronize(c->own_stream), "clear counters")) {
+        (void)hipFree(counters);
+        delete c;
+        return nullptr;
+    }
+    c->counters = static_cast<int *>(counters);
+    c->counter_bytes = c->prefill_counter_bytes = kFirstCounters * sizeof(int);
     // The allocation-free decode's fixed partials array: its address on this
     // device is taken here, once, so that entry point's first call loads
     // nothing.
@@ -676,7 +697,18 @@ int mslim_attn_prefill_causal(void *ctx, const void *q, const void *k, const voi
     l.head_dim = head_dim; l.scale = scale;
     l.split_allowed = c.prefill_split;
     l.pool_allowed = c.prefill_pool;
-    const mslim::PrefillSplit plan = mslim::prefill_split_plan(l);
+    mslim::PrefillSplit plan = mslim::prefill_split_plan(l);
+    if (plan.chunk_tiles && mslim::prefill_wide(l) &&
+        (plan.partial_bytes > c.prefill_partial_bytes || plan.counters * sizeof(int) > c.prefill_counter_bytes)) {
+        // These groups are accepted under capture with no call before: there
+        // nothing can be allocated, so the launch runs unsplit.
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (int rc = check_hip(hipStreamIsCapturing(c.stream, &capture), "hipStreamIsCapturing")) return rc;
+        if (capture != hipStreamCaptureStatusNone) {
+            l.split_allowed = false;
+            plan = mslim::prefill_split_plan(l);
+        }
+    }
     const int pool = plan.chunk_tiles ? 0 : mslim::prefill_pool_items(l);
     if (plan.chunk_tiles || pool) {
         if (plan.chunk_tiles) {

@@ -93,6 +93,8 @@ struct PrefillLaunch {
 };
 // True when the MFMA kernel covers this launch (geometry and alignment).
 bool prefill_mfma(const PrefillLaunch &l);
+// True when it does so in its WIDE form (groups other than 1, 2 and multiples of 4).
+bool prefill_wide(const PrefillLaunch &l);
 // Row blocks per XCD that an unsplit launch hands out at run time (0: none).
 int prefill_pool_items(const PrefillLaunch &l);
 // How a launch splits its row blocks: chunk_tiles == 0 means no split.

@@ -838,6 +838,8 @@ bool prefill_mfma(const PrefillLaunch &l) {
     return (loads & 15) == 0 && (reinterpret_cast<uintptr_t>(l.out) & 7) == 0;
 }
 
+bool prefill_wide(const PrefillLaunch &l) { return prefill_mfma(l) && !even_group(l.q_heads / l.kv_heads); }
+
 namespace {
 
 // Predicted span, in 64-key tiles, of a launch whose row blocks split into
