@@ -930,7 +930,7 @@ def main() -> int:
             "unit": "GB/s",
             "ms": round(seal_ms, 4),
             "records": total_pages,
-            "kernel": "token_hashes_kernel + frame_kernel: ColdStore record frames (header, per-token "
+            "kernel": "token_hashes_kernel + payload_sums_kernel + frame_kernel: ColdStore record frames (header, per-token "
                       "FNV tables, record FNV, SHA-256) of every cfg4 pool page; value = K+V payload "
                       "bytes sealed per second",
         },
