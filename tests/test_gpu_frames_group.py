@@ -79,3 +79,24 @@ def test_group_kernel_ignores_what_follows_the_last_token(ctx):
     ctx.frames_decode(q, kv[0], F16, kv[1], F16, out, tokens, qh, kvh, d)
     torch.cuda.synchronize()
     assert torch.equal(clean, out) and torch.isfinite(out).all()
+
+
+@pytest.mark.parametrize("tokens,dead", [(65, [64]), (65, list(range(64))), (300, [0, 5, 130, 299]), (9, [3])])
+@pytest.mark.parametrize("qh,kvh,d", [(32, 8, 128), (3, 3, 64), (8, 1, 136)])
+def test_keys_at_minus_infinity_weigh_nothing(ctx, qh, kvh, d, tokens, dead):
+    # A key whose scores are all -inf has probability zero, also where it is
+    # the first or only key that a lane group, a wavefront or a split meets:
+    # the output is that of the other keys.  With fewer than 300 keys left,
+    # |score| < 16 and |v| < 6, test_group_kernel's bound is below 6e-4.
+    gen = torch.Generator(device="cuda").manual_seed(tokens + d)
+    q = torch.rand((qh, d), generator=gen, device="cuda") + 0.25
+    k, v = (torch.randn((tokens, kvh, d), generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2))
+    live = [t for t in range(tokens) if t not in dead]
+    k[dead] = -float("inf")
+    out = torch.empty_like(q)
+    ctx.frames_decode(q, k, BF16, v, BF16, out, tokens, qh, kvh, d)
+    group = qh // kvh
+    kl, vl = (x[live].double().repeat_interleave(group, dim=1) for x in (k, v))
+    p = torch.softmax((kl * q.double()).sum(dim=2) * d ** -0.5, dim=0)
+    ref = (p[:, :, None] * vl).sum(dim=0)
+    assert (out.double() - ref).abs().max() <= 6e-4

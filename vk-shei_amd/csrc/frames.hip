@@ -380,15 +380,18 @@ __global__ __launch_bounds__(kThreads) void frames_group_kernel(FramesArgs a) {
             float m_new = m[g];
 #pragma unroll
             for (int u = 0; u < kSteps; ++u) m_new = fmaxf(m_new, s[u][g]);
-            // a row group without a token so far keeps m = -inf, l = 0
+            // A row group that has met no score above -inf keeps m = -inf and
+            // l = 0: a score of -inf (a row past the split, or a key's own)
+            // weighs nothing whatever the base.
             const float alpha = m_new == m[g] ? 1.0f : __builtin_amdgcn_exp2f(m[g] - m_new);
+            const float base = m_new == -INFINITY ? 0.0f : m_new;
             m[g] = m_new;
             l[g] *= alpha;
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc[g][e] *= alpha;
 #pragma unroll
             for (int u = 0; u < kSteps; ++u) {
-                s[u][g] = t0 + u * RPI + lr < end ? __builtin_amdgcn_exp2f(s[u][g] - m_new) : 0.0f;
+                s[u][g] = t0 + u * RPI + lr < end ? __builtin_amdgcn_exp2f(s[u][g] - base) : 0.0f;
                 l[g] += s[u][g];
             }
         }
@@ -432,7 +435,7 @@ __global__ __launch_bounds__(kThreads) void frames_group_kernel(FramesArgs a) {
         for (int i = 0; i < PARTS; ++i) mx = fmaxf(mx, ml_lds[i][g][0]);
 #pragma unroll
         for (int i = 0; i < PARTS; ++i) {
-            // l = 0: no token reached this part (a token's own p is 1 or NaN)
+            // l = 0: every score of this part was -inf, or it had no token
             const float w = ml_lds[i][g][1] == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(ml_lds[i][g][0] - mx);
             sum = fmaf(w, ml_lds[i][g][1], sum);
             const float4 x = *reinterpret_cast<const float4 *>(&acc_lds[i][g][d]);
@@ -492,7 +495,7 @@ __global__ __launch_bounds__(kThreads) void frames_group_kernel(FramesArgs a) {
 #pragma unroll
             for (int j = 0; j < kBatch; ++j) {
                 if (s0 + j * ways < a.splits) {
-                    const float w = __builtin_amdgcn_exp2f(ml[j].x - mx);
+                    const float w = ml[j].y == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(ml[j].x - mx);
                     sum = fmaf(w, ml[j].y, sum);
                     o.x = fmaf(w, x0[j].x, o.x); o.y = fmaf(w, x0[j].y, o.y);
                     o.z = fmaf(w, x1[j].x, o.z); o.w = fmaf(w, x1[j].y, o.w);
