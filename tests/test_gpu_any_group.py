@@ -151,3 +151,54 @@ def test_prefill_first_call_under_capture():
         del graph
     finally:
         fresh.close()
+
+
+def _attend64(q, k, v, group):
+    """q [n][qh][d] attends k, v [t][kvh][d], causal at the end, in float64.
+    A key whose score is -inf weighs nothing."""
+    n, t = q.shape[0], k.shape[0]
+    kl, vl = (x.double().repeat_interleave(group, dim=1) for x in (k, v))
+    score = torch.einsum("nhd,thd->nht", q.double().cpu(), kl.cpu()) * q.shape[2] ** -0.5
+    seen = torch.arange(t)[None, :] <= torch.arange(n)[:, None] + (t - n)
+    score.masked_fill_(~seen[:, None, :], -float("inf"))
+    p = torch.softmax(score, dim=2)
+    out = torch.zeros(q.shape, dtype=torch.float64)
+    for i in range(n):  # only the keys that the row sees and weighs
+        for h in range(q.shape[1]):
+            keys = (p[i, h] > 0).nonzero()[:, 0]
+            out[i, h] = (p[i, h, keys, None] * vl[keys, h].cpu()).sum(dim=0) if len(keys) else float("nan")
+    return out
+
+
+def _check64(got, ref, label):
+    # the bound above with |v| < 6, where the reference is finite; elsewhere
+    # the same infinity or NaN
+    got, finite = got.double().cpu(), torch.isfinite(ref)
+    assert torch.equal(torch.nan_to_num(got[~finite], nan=7.0), torch.nan_to_num(ref[~finite], nan=7.0)), label
+    over = (got - ref).abs()[finite] > ref.abs()[finite] * 2.0 ** -8 + 6 * 2.0 ** -13
+    assert not over.any(), (label, int(over.sum()))
+
+
+@pytest.mark.parametrize("qh,kvh,d", [(3, 1, 128), (10, 2, 64), (14, 2, 128)])
+@pytest.mark.parametrize("queries,prior,values,dead", [(90, 0, [40, 89], []), (300, 0, [130, 299], [64]),
+                                                       (64, 1500, [1530], [1500]), (65, 0, [], [0, 64])])
+def test_prefill_any_group_values_that_are_not_finite(ctx, qh, kvh, d, queries, prior, values, dead):
+    # An infinity or NaN of V reaches the rows that see its key, in its own
+    # dimension, and no earlier row; a key at -inf weighs nothing.
+    gen = torch.Generator(device="cuda").manual_seed(queries + d)
+    t = queries + prior
+    q = (torch.rand((queries, qh, d), generator=gen, device="cuda") + 0.25).to(torch.bfloat16)
+    k, v = (torch.randn((t, kvh, d), generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2))
+    k[dead] = -float("inf")
+    for i in values:
+        v[i, :, 3], v[i, :, 17], v[i, :, d - 1] = float("inf"), -float("inf"), float("nan")
+    ref = _attend64(q, k, v, qh // kvh)
+    split, unsplit = torch.empty_like(q), torch.empty_like(q)
+    ctx.prefill_causal(q, k, v, split, queries, prior, qh, kvh, d)
+    try:
+        ctx.set_prefill_split(False)
+        ctx.prefill_causal(q, k, v, unsplit, queries, prior, qh, kvh, d)
+    finally:
+        ctx.set_prefill_split(True)
+    _check64(split, ref, "split")
+    _check64(unsplit, ref, "unsplit")

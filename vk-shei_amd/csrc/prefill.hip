@@ -117,6 +117,14 @@ struct Swz {
     }
 };
 
+// The kernel arguments read anew, for code off the main path: values that it
+// took from the loads of the main path would hold scalar registers there.
+__device__ __forceinline__ const PrefillArgs *reread_args() {
+    uint64_t base = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(base));
+    return reinterpret_cast<const PrefillArgs *>(base);
+}
+
 // Iteration j of a wavefront issues the QK MFMAs of tile j, then the P.V
 // MFMAs of tile j-1 with the softmax of tile j spread over their slots (row
 // maximum in the first two slots, exp2 / BF16 pack / row sums in the rest).
@@ -624,7 +632,56 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
     else pv_softmax(3, Yes{}, No{}, No{});
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // no DMA may still target LDS at exit
 
-    const float l = l_run + __shfl_xor(l_run, 32, 64);
+    float l = l_run + __shfl_xor(l_run, 32, 64);
+    if constexpr (WIDE) {
+        // An infinity or NaN of V meets every row of its tile in the P.V
+        // MFMAs: 0 x Inf where the row masks the key, and Inf + 0 x Inf where
+        // a p has no low part.  A score of -inf has no maximum to be relative
+        // to when it is a chunk's only one.  Rows that end up without a finite
+        // sum are taken again key by key in f32 over the keys they see, as
+        // the any-geometry kernel does (a sum of zeros is zero, so a finite
+        // row costs an FMA per value, once per workgroup).
+        float chain[8] = {l * 0.0f};
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) chain[r % 8] = fmaf(o[mt][r], 0.0f, chain[r % 8]);
+        float probe = ((chain[0] + chain[1]) + (chain[2] + chain[3])) + ((chain[4] + chain[5]) + (chain[6] + chain[7]));
+        probe += __shfl_xor(probe, 32, 64);
+        if (__builtin_expect(probe != 0.0f && row < a.queries, 0)) {
+            const PrefillArgs &z = *reread_args();
+            const int first_key = tb * kBN, past_key = min(te * kBN, z.prior + row + 1);
+            const int64_t stride = (int64_t)z.kv_heads * D;
+            const uint16_t *qp = z.q + ((int64_t)row * z.q_heads + head) * D;
+            const uint16_t *kp = z.k + (int64_t)kvh * D, *vp = z.v + (int64_t)kvh * D + half * 4;
+            auto score = [&](int t) __attribute__((always_inline)) {
+                float dot = 0.0f;
+#pragma unroll 1
+                for (int d = 0; d < D; ++d) dot = fmaf(read_bf16(qp[d]), read_bf16(kp[t * stride + d]), dot);
+                return dot;
+            };
+            float m = -INFINITY;
+#pragma unroll 1
+            for (int t = first_key; t < past_key; ++t) m = fmaxf(m, score(t));
+            m_used = m * z.scale_log2e;
+            l = 0.0f;
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[mt][r] = 0.0f;
+#pragma unroll 1
+            for (int t = first_key; t < past_key; ++t) {
+                const float x = score(t);
+                const float p = x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(fmaf(x, z.scale_log2e, -m_used));
+                l += p;
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        o[mt][r] = fmaf(p, read_bf16(vp[t * stride + mt * 32 + r / 4 * 8 + r % 4]), o[mt][r]);
+            }
+        }
+    }
     // O / l as O * (1 / l): one correctly rounded reciprocal per row instead
     // of D divisions (within one f32 ulp of the quotient before the BF16
     // rounding).
