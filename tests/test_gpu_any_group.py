@@ -179,6 +179,27 @@ def _check64(got, ref, label):
     assert not over.any(), (label, int(over.sum()))
 
 
+@pytest.mark.parametrize("qh,kvh,d", [(3, 1, 128), (10, 2, 72), (12, 4, 64)])
+@pytest.mark.parametrize("t,values,dead", [(33, [32], []), (300, [0, 150], []), (257, [256], [255]), (33, [], [32]),
+                                           (300, [7], list(range(64, 128)))])
+def test_decode_any_group_values_that_are_not_finite(ctx, qh, kvh, d, t, values, dead):
+    # values: tokens whose V row holds +Inf, -Inf and NaN in three dimensions;
+    # dead: keys at -inf, alone in a wavefront's tile or filling a partition.
+    # Rows past the sequence hold NaN and must not be read into the result.
+    gen = torch.Generator(device="cuda").manual_seed(t + d)
+    q = (torch.rand((1, qh, d), generator=gen, device="cuda") + 0.25).to(torch.bfloat16)
+    k, v = (torch.randn((t + 64, kvh, d), generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2))
+    k[dead] = -float("inf")
+    for i in values:
+        v[i, :, 3], v[i, :, 17], v[i, :, d - 1] = float("inf"), -float("inf"), float("nan")
+    k[t:], v[t:] = float("nan"), float("nan")
+    ref = _attend64(q, k[:t], v[:t], qh // kvh)
+    for split in (0, 64):
+        out = torch.empty_like(q)
+        ctx.decode_dense(q, k, v, out, [t], qh, kvh, d, seq_stride_tokens=t + 64, split_tokens=split)
+        _check64(out, ref, f"split {split}")
+
+
 @pytest.mark.parametrize("qh,kvh,d", [(3, 1, 128), (10, 2, 64), (14, 2, 128)])
 @pytest.mark.parametrize("queries,prior,values,dead", [(90, 0, [40, 89], []), (300, 0, [130, 299], [64]),
                                                        (64, 1500, [1530], [1500]), (65, 0, [], [0, 64])])

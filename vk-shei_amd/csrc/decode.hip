@@ -127,6 +127,14 @@ __device__ __forceinline__ Tables tables_of(const DeviceArgs &a) {
     return t;
 }
 
+// The kernel arguments read anew, for code off the main path: values that it
+// took from the loads of the main path would hold scalar registers there.
+__device__ __forceinline__ const DeviceArgs *reread_args() {
+    uint64_t base = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(base));
+    return reinterpret_cast<const DeviceArgs *>(base);
+}
+
 // Base of the 16-token block starting at logical token t0 (a multiple of 16).
 template <bool PAGED>
 __device__ __forceinline__ const uint16_t *block_base(const DeviceArgs &a, const uint16_t *cache,
@@ -464,6 +472,71 @@ __global__ __launch_bounds__(64 * kWaves, 2) void decode_kernel(DeviceArgs a) {
     // heads 4*grp + i, dims 16*slice + row16.
     l_run = wave_xor_sum(l_run, 16);
     l_run = wave_xor_sum(l_run, 32);
+    if constexpr (G == 0) {
+        // An infinity or NaN of V turns into NaN in the P.V MFMAs where a p is
+        // zero (a token past the end repeats the last row, a p without a low
+        // part), and a tile whose scores are all -inf has no maximum to be
+        // relative to.  A wavefront that ends up with a value that is not
+        // finite takes its tiles again token by token in f32, as the
+        // any-geometry kernel does (a sum of zeros is zero, so finite values
+        // cost an FMA each, once per partition).
+        floatx4_t probe = {l_run * 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int sl = 0; sl < NS; ++sl)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) probe[i] = fmaf(o[sl][i], 0.0f, probe[i]);
+        if (__builtin_expect(wave_any((probe[0] + probe[1]) + (probe[2] + probe[3]) != 0.0f), 0)) {
+            const DeviceArgs &r = *reread_args();
+            const int rn = group_of<G>(r), rd = dim_of<D, G>(r);
+            const int r_begin = split * r.split_tokens;
+            const int r_end = min(tables_of(r).seq_len(b), r_begin + r.split_tokens);
+            auto row_of = [&](const uint16_t *cache, int t) __attribute__((always_inline)) {
+                return block_base<PAGED>(r, cache, b, kvh, t & ~15, rd) + (t & 15) * row_stride<PAGED>(r, rd);
+            };
+#pragma unroll 1
+            for (int h = 0; h < rn; ++h) {
+                const uint16_t *qp = r.q + ((int64_t)b * r.q_heads + kvh * rn + h) * rd;
+                auto score = [&](int t) __attribute__((always_inline)) {
+                    const uint16_t *kp = row_of(r.k, t);
+                    float dot = 0.0f;
+                    for (int d = lane; d < rd; d += 64) dot = fmaf(read_bf16(qp[d]), read_bf16(kp[d]), dot);
+#pragma unroll 1
+                    for (int mask = 1; mask < 64; mask <<= 1) dot = wave_xor_sum(dot, mask);
+                    return dot;
+                };
+                // the tokens of this wavefront's tiles, in order
+                auto next = [&](int t) __attribute__((always_inline)) {
+                    return (t + 1 - r_begin) % kTile ? t + 1 : t + 1 + (kWaves - 1) * kTile;
+                };
+                // the lowest finite maximum where every score is -inf: the
+                // merges weigh that part's l = 0 with exp2 of a difference
+                float m = -__FLT_MAX__, l = 0.0f, acc[NS] = {};
+#pragma unroll 1
+                for (int t = r_begin + wave * kTile; t < r_end; t = next(t)) m = fmaxf(m, score(t));
+#pragma unroll 1
+                for (int t = r_begin + wave * kTile; t < r_end; t = next(t)) {
+                    const float x = score(t);
+                    const float p = x == -INFINITY ? 0.0f
+                                                   : __builtin_amdgcn_exp2f(fmaf(x, r.scale_log2e, -m * r.scale_log2e));
+                    l += p;
+                    const uint16_t *vp = row_of(r.v, t);
+#pragma unroll
+                    for (int sl = 0; sl < NS; ++sl)
+                        if (sl * 16 + row16 < rd) acc[sl] = fmaf(p, read_bf16(vp[sl * 16 + row16]), acc[sl]);
+                }
+                if (row16 == h) {
+                    m_run = m;
+                    l_run = l;
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (4 * grp + i == h) {
+#pragma unroll
+                        for (int sl = 0; sl < NS; ++sl) o[sl][i] = acc[sl];
+                    }
+            }
+        }
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int h = 4 * grp + i;
