@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -278,10 +279,20 @@ int frames_enqueue(Context &c, mslim::FramesLaunch &l, uint64_t *scratch) {
     *scratch = 0;
     l.scale = (float)(1.0 / std::sqrt((double)l.head_dim));
     l.split_tokens = l.tokens > 0 ? mslim::frames_split_tokens(l) : 256;
-    const int64_t splits = (l.tokens + l.split_tokens - 1) / l.split_tokens;
+    int64_t splits = (l.tokens + l.split_tokens - 1) / l.split_tokens;
+    auto bytes_of = [&](int64_t floats) { return (size_t)l.q_heads * splits * floats * sizeof(float); };
+    if (splits > 1 && bytes_of(2 + l.head_dim) > c.workspace_bytes && l.tokens <= INT_MAX && mslim::frames_grouped(l)) {
+        // Short caches are accepted under capture with no call before: there
+        // nothing can be allocated, so the launch runs unsplit.
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (int rc = check_hip(hipStreamIsCapturing(c.stream, &capture), "hipStreamIsCapturing")) return rc;
+        if (capture != hipStreamCaptureStatusNone) {
+            l.split_tokens = (int)l.tokens;
+            splits = 1;
+        }
+    }
     if (splits > 1) {
-        const size_t ml = (size_t)l.q_heads * splits * 2 * sizeof(float);
-        const size_t acc = (size_t)l.q_heads * splits * l.head_dim * sizeof(float);
+        const size_t ml = bytes_of(2), acc = bytes_of(l.head_dim);
         if (int rc = grow_device(c, &c.workspace, &c.workspace_bytes, ml + acc,
                                  "hipMalloc frames split workspace"))
             return rc;
@@ -353,8 +364,7 @@ void *mslim_attn_ctx_new(void) {
     }
     c->proj_partial_bytes = mslim::kProjPartialBytes;
     // Counters of fused merges and of pooled prefill, zero from here on: the
-    // portable decode never needs more, nor does a prefill that runs unsplit,
-    // so their first call may be under capture too.
+    // portable decode never needs more, nor does a prefill that runs unsplit.
     void *counters = nullptr;
     if (check_hip(hipMalloc(&counters, kFirstCounters * sizeof(int)), "hipMalloc split counters") ||
         check_hip(hipMalloc(&c->prefill_counters, kFirstCounters * sizeof(int)), "hipMalloc prefill counters") ||
