@@ -105,10 +105,27 @@ int mslim_attn_check_bf16_encoding(void *ctx, uint64_t *mismatches);
  * single queue (gpu_resources.rs:122-123); callers that share a stream with
  * other libraries need to name it. */
 int mslim_attn_ctx_set_stream(void *ctx, void *hip_stream);
-/* A context's decode workspace and split counters serve one stream at a
- * time: mslim_attn_ctx_set_stream waits for the work queued on the old
- * stream before it switches, and one context must not be driven from two
- * host threads on two streams at once. */
+/* A context's workspaces and split counters serve one stream at a time:
+ * mslim_attn_ctx_set_stream waits for the work queued on the old stream
+ * before it switches, and one context must not be driven from two host
+ * threads on two streams at once.
+ *
+ * Calls recorded into a graph.  A recorded call keeps the addresses of the
+ * context buffers that it uses: decode and its portable form their split
+ * partials and counters, a prefill its split partials or pool counter,
+ * products of more than 16 token rows their split partials, the fused RMSNorm
+ * entry points their normalised and Q/K/V rows, RoPE its cos/sin table.
+ *   * The addresses stay valid until mslim_attn_ctx_destroy: a call that needs
+ *     a larger buffer keeps the replaced one.  Destroy graphs first.
+ *   * A replay is one more user of those buffers, so it takes its place in the
+ *     context's one-stream order: a replay that overlaps another call on the
+ *     context, or another graph recorded on it, can give wrong results.
+ *     Graphs that must overlap are recorded on contexts of their own.
+ *   * A RoPE call recorded with one configuration (head_dim, theta, scaling)
+ *     is not replayed after the context ran another.
+ *   * Nothing can be allocated while recording.  A call whose buffers are not
+ *     there yet fails, except where it can run without: a prefill of a group
+ *     other than 1, 2 or a multiple of 4 and a portable decode run unsplit. */
 
 /* Context options.  No reference counterpart (the OpenCL engine has no merge
  * choice); for tests and callers that want the two-launch merge.

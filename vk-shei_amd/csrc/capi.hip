@@ -84,11 +84,16 @@ struct Context {
     hipEvent_t ev_start = nullptr, ev_end = nullptr;
     void *gemm_in = nullptr, *gemm_out = nullptr;  // device staging of matrix_multiply
     size_t gemm_in_bytes = 0, gemm_out_bytes = 0;
+    // Buffers that a larger one took the place of (grow_recorded)
+    static constexpr int kMaxRetired = 256;
+    void *retired[kMaxRetired];
+    int retired_count = 0;
 
     ~Context() {
         if (stream) (void)hipStreamSynchronize(stream);
         if (gemm_in) (void)hipFree(gemm_in);
         if (gemm_out) (void)hipFree(gemm_out);
+        for (int i = 0; i < retired_count; ++i) (void)hipFree(retired[i]);
         if (workspace) (void)hipFree(workspace);
         if (swiglu_table) (void)hipFree(swiglu_table);
         if (proj_partial) (void)hipFree(proj_partial);
@@ -114,8 +119,31 @@ struct Context {
 
 Context *ctx_of(void *handle) { return static_cast<Context *>(handle); }
 
-// Grow a device scratch buffer; the stream is drained first so no queued
-// kernel still uses the old allocation.
+// Grow a device buffer whose address a graph may have recorded, or a queued
+// kernel may still use: the old one stays allocated until the context goes.
+// A new buffer has at least twice the old one's bytes, so all that are kept
+// take less than the one in use; only where that much cannot be had is it
+// exactly as large as asked.
+int grow_recorded(Context &c, void **mem, size_t *cap, size_t bytes, const char *what) {
+    if (*cap >= bytes) return 0;
+    if (c.retired_count == Context::kMaxRetired) return fail(std::string(what) + ": buffer replaced too often", 100);
+    void *fresh = nullptr;
+    size_t size = std::max(bytes, 2 * *cap);
+    hipError_t e = hipMalloc(&fresh, size);
+    if (e != hipSuccess && size > bytes) {
+        (void)hipGetLastError();
+        size = bytes;
+        e = hipMalloc(&fresh, size);
+    }
+    if (int rc = check_hip(e, what)) return rc;
+    if (*mem) c.retired[c.retired_count++] = *mem;
+    *mem = fresh;
+    *cap = size;
+    return 0;
+}
+
+// Grow a device buffer that no recorded call uses; the stream is drained
+// first so no queued kernel still uses the old allocation.
 int grow_device(Context &c, void **mem, size_t *cap, size_t bytes, const char *what) {
     if (*cap >= bytes) return 0;
     if (*mem) {
@@ -206,7 +234,7 @@ constexpr int kFirstCounters = 2048;
 int split_counters(Context &c, size_t n) {
     if (c.counter_bytes < n * sizeof(int)) {
         void *mem = c.counters;
-        if (int rc = grow_device(c, &mem, &c.counter_bytes, n * sizeof(int), "hipMalloc split counters")) return rc;
+        if (int rc = grow_recorded(c, &mem, &c.counter_bytes, n * sizeof(int), "hipMalloc split counters")) return rc;
         c.counters = static_cast<int *>(mem);
         c.counters_dirty = true;
     }
@@ -222,8 +250,8 @@ int split_counters(Context &c, size_t n) {
 
 int decode_common(Context &c, mslim::DecodeLaunch &l, const int32_t *seq_lens, int split_tokens) {
     if (int rc = decode_prepare(l, seq_lens, split_tokens)) return rc;
-    if (int rc = grow_device(c, &c.workspace, &c.workspace_bytes, mslim::decode_partial_bytes(l),
-                             "hipMalloc decode split workspace"))
+    if (int rc = grow_recorded(c, &c.workspace, &c.workspace_bytes, mslim::decode_partial_bytes(l),
+                               "hipMalloc decode split workspace"))
         return rc;
     decode_place_partials(l, c.workspace);
     // One split counter per (sequence, kv head).
@@ -293,8 +321,8 @@ int frames_enqueue(Context &c, mslim::FramesLaunch &l, uint64_t *scratch) {
     }
     if (splits > 1) {
         const size_t ml = bytes_of(2), acc = bytes_of(l.head_dim);
-        if (int rc = grow_device(c, &c.workspace, &c.workspace_bytes, ml + acc,
-                                 "hipMalloc frames split workspace"))
+        if (int rc = grow_recorded(c, &c.workspace, &c.workspace_bytes, ml + acc,
+                                   "hipMalloc frames split workspace"))
             return rc;
         l.partial_ml = static_cast<float *>(c.workspace);
         l.partial_acc = reinterpret_cast<float *>(static_cast<char *>(c.workspace) + ml);
@@ -722,16 +750,16 @@ int mslim_attn_prefill_causal(void *ctx, const void *q, const void *k, const voi
     const int pool = plan.chunk_tiles ? 0 : mslim::prefill_pool_items(l);
     if (plan.chunk_tiles || pool) {
         if (plan.chunk_tiles) {
-            if (int rc = grow_device(c, &c.prefill_partial, &c.prefill_partial_bytes, plan.partial_bytes,
-                                     "hipMalloc prefill split partials"))
+            if (int rc = grow_recorded(c, &c.prefill_partial, &c.prefill_partial_bytes, plan.partial_bytes,
+                                       "hipMalloc prefill split partials"))
                 return rc;
         }
         // A split launch counts chunks per row block; a pooled one draws
         // from counter 0.  Both leave their counters at zero.
         const size_t ctr_bytes = plan.chunk_tiles ? (size_t)plan.counters * sizeof(int) : sizeof(int);
         if (c.prefill_counter_bytes < ctr_bytes) {
-            if (int rc = grow_device(c, &c.prefill_counters, &c.prefill_counter_bytes, ctr_bytes,
-                                     "hipMalloc prefill split counters"))
+            if (int rc = grow_recorded(c, &c.prefill_counters, &c.prefill_counter_bytes, ctr_bytes,
+                                       "hipMalloc prefill split counters"))
                 return rc;
             c.prefill_counters_dirty = true;
         }
@@ -877,25 +905,14 @@ static mslim::RopeCosSin rope_cossin(Context &c, int head_dim, float theta, int 
     if (same) want = std::max(want, c.rope_positions);
     const size_t bytes = (size_t)want * row_bytes;
     if (bytes > c.rope_bytes) {
-        // work queued on the stream may still read the old table
-        if (c.rope_rows) {
-            if (hipStreamSynchronize(c.stream) != hipSuccess || hipFree(c.rope_rows) != hipSuccess) {
-                (void)hipGetLastError();
-                c.rope_rows = nullptr;
-                c.rope_bytes = 0;
-                c.rope_positions = 0;
-                return {};
-            }
-        }
-        c.rope_rows = nullptr;
-        c.rope_bytes = 0;
-        c.rope_positions = 0;
-        if (hipMalloc(reinterpret_cast<void **>(&c.rope_rows), bytes) != hipSuccess) {
+        void *rows = c.rope_rows;
+        if (grow_recorded(c, &rows, &c.rope_bytes, bytes, "hipMalloc RoPE table")) {
             (void)hipGetLastError();
-            c.rope_rows = nullptr;
+            g_error.clear();
             return {};
         }
-        c.rope_bytes = bytes;
+        c.rope_rows = static_cast<uint16_t *>(rows);
+        c.rope_positions = 0;
     }
     if (mslim::launch_rope_cossin(c.rope_rows, want, head_dim, theta, llama3, factor, low, high, original_max,
                                   c.stream) != hipSuccess) {
@@ -1335,7 +1352,7 @@ static int proj_partials(Context &c, std::initializer_list<int> rows, int produc
     *partial = nullptr;
     const size_t floats = mslim::proj_partial_floats(rows.begin(), (int)rows.size(), products, inner, tokens);
     if (!floats) return 0;
-    if (grow_device(c, &c.proj_partial, &c.proj_partial_bytes, floats * sizeof(float), "hipMalloc projection partials"))
+    if (grow_recorded(c, &c.proj_partial, &c.proj_partial_bytes, floats * sizeof(float), "hipMalloc projection partials"))
         return 400;
     *partial = static_cast<float *>(c.proj_partial);
     return 0;
@@ -1493,7 +1510,7 @@ int mslim_attn_gemm_qkv(void *ctx, const void *q_weight, const void *k_weight, c
 // not normalise themselves): mslim_attn_rmsnorm's kernels.
 static int normalise_rows(Context &c, const void *input, const void *norm_weight, float epsilon, int inner,
                           int tokens, const void **rows) {
-    if (grow_device(c, &c.norm_rows, &c.norm_rows_bytes, (size_t)inner * tokens * 2, "hipMalloc normalised rows"))
+    if (grow_recorded(c, &c.norm_rows, &c.norm_rows_bytes, (size_t)inner * tokens * 2, "hipMalloc normalised rows"))
         return 400;
     if (int rc = check_hip(mslim::launch_rmsnorm(static_cast<const uint16_t *>(input),
                                                  static_cast<const uint16_t *>(norm_weight),
@@ -1671,7 +1688,7 @@ int mslim_attn_rmsnorm_qkv_rope_append(void *ctx, const void *norm_weight, float
     // under the one lock (another call on the context may not regrow the
     // buffer in between).
     const size_t bytes = (size_t)batch * (q_rows + 2 * (size_t)kv_rows) * 2;
-    if (grow_device(c, &c.qkv_rows, &c.qkv_rows_bytes, bytes, "hipMalloc QKV rows")) return 400;
+    if (grow_recorded(c, &c.qkv_rows, &c.qkv_rows_bytes, bytes, "hipMalloc QKV rows")) return 400;
     uint16_t *q = static_cast<uint16_t *>(c.qkv_rows);
     uint16_t *k = q + (size_t)batch * q_rows, *v = k + (size_t)batch * kv_rows;
     if (int rc = rmsnorm_gemm_qkv_locked(c, norm_weight, epsilon, q_weight, k_weight, v_weight, input, q, k, v, inner,
