@@ -125,7 +125,8 @@ int mslim_attn_ctx_set_stream(void *ctx, void *hip_stream);
  *     is not replayed after the context ran another.
  *   * Nothing can be allocated while recording.  A call whose buffers are not
  *     there yet fails, except where it can run without: a prefill of a group
- *     other than 1, 2 or a multiple of 4 and a portable decode run unsplit. */
+ *     other than 1, 2 or a multiple of 4 and a portable decode run unsplit,
+ *     and so do products, to the same bits. */
 
 /* Context options.  No reference counterpart (the OpenCL engine has no merge
  * choice); for tests and callers that want the two-launch merge.
@@ -535,9 +536,10 @@ int mslim_attn_matrix_multiply(void *ctx, const void *weight, const uint8_t *inp
  * :553-596); larger products run on the tiled MFMA kernel of the prompt
  * chunks (llm_prefill_gemv_reuse8/16/32, gpu_llm.cl:553-683), or, for inner
  * not a multiple of 64 or unaligned buffers, a kernel of one wavefront per
- * output.  Each product of a given shape is summed in one fixed order, so
+ * output.  Each of the three sums a matrix's products in one fixed order, so
  * every entry point below that fuses an epilogue gives the same bits as this
- * one followed by the elementwise call. */
+ * one followed by the elementwise call, and a token row of a call of more than
+ * 16 rows has the same bits whatever other rows share the call. */
 int mslim_attn_gemm_bf16(void *ctx, const void *weight, const void *input, void *output, int inner,
                          int rows, int tokens);
 

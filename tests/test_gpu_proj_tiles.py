@@ -58,3 +58,33 @@ def test_projection_tiles(ctx, inner, rows, kv_rows, tokens):
     ctx.swiglu(k1, up, act, tokens * kv_rows)
     ctx.gemm_swiglu(wk, wv, x, swiglu, inner, kv_rows, tokens)
     assert same(swiglu, act)
+
+
+# (inner, rows of Q, rows of K and V): one, two, four and eight k segments, and
+# K and V with other counts than their Q.
+@pytest.mark.parametrize("inner,rows,kv_rows", [(4096, 4096, 1024), (14336, 4096, 4096), (8192, 2048, 512),
+                                                (2048, 9000, 2048), (1024, 4096, 256), (8192, 8192, 1024)])
+def test_a_rows_bits_do_not_depend_on_its_launch(ctx, inner, rows, kv_rows):
+    # every row count of more than 16 gives a token row the bits it has among
+    # 512 rows, in the plain, residual, SwiGLU and Q-K-V products
+    gen = torch.Generator(device="cuda").manual_seed(inner + rows)
+
+    def normal(shape, scale):
+        return (torch.randn(shape, generator=gen, device="cuda") * scale).to(torch.bfloat16)
+
+    x, wq, wk, wv = (normal(s, c) for s, c in (((512, inner), 1.0), ((rows, inner), 0.02), ((kv_rows, inner), 0.02),
+                                               ((kv_rows, inner), 0.02)))
+
+    def products(t):
+        plain, add, swiglu, q, k, v = (torch.full((t, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+                                       for n in (rows, rows, kv_rows, rows, kv_rows, kv_rows))
+        ctx.gemm_bf16(wq, x, plain, inner, rows, t)
+        ctx.gemm_bf16_add(wq, x, plain, add, inner, rows, t)
+        ctx.gemm_swiglu(wk, wv, x, swiglu, inner, kv_rows, t)
+        ctx.gemm_qkv(wq, wk, wv, x, q, k, v, inner, rows, kv_rows, t)
+        return [y.view(torch.int16) for y in (plain, add, swiglu, q, k, v)]
+
+    want = products(512)
+    for t in (17, 32, 64, 65, 100, 120, 128, 129, 200, 250, 256, 257, 300, 400, 511):
+        for got, ref in zip(products(t), want):
+            assert torch.equal(got, ref[:t]), t

@@ -126,3 +126,19 @@ def test_replay_after_a_larger_call(fresh, name):
     big_call(big_again)
     torch.cuda.synchronize()
     assert torch.equal(big, big_again)
+
+
+@pytest.mark.parametrize("inner,rows,tokens", [(4096, 4096, 32), (14336, 4096, 64), (8192, 2048, 300)])
+def test_product_first_call_under_capture(fresh, inner, rows, tokens):
+    # Run eagerly these split along k; with nothing allocated for the partials
+    # the recorded call adds its segments in registers, to the same bits.
+    call, want = _product(fresh, inner, rows, tokens)
+    got = torch.zeros_like(want)
+    graph = _record(fresh, lambda: call(got))
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        call(want)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)

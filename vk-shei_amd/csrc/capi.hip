@@ -384,13 +384,6 @@ void *mslim_attn_ctx_new(void) {
         delete c;
         return nullptr;
     }
-    // Partials of split projections, enough for every shape of inner < 8192:
-    // those calls allocate nothing, so their first one may be under capture.
-    if (check_hip(hipMalloc(&c->proj_partial, mslim::kProjPartialBytes), "hipMalloc projection partials")) {
-        delete c;
-        return nullptr;
-    }
-    c->proj_partial_bytes = mslim::kProjPartialBytes;
     // Counters of fused merges and of pooled prefill, zero from here on: the
     // portable decode never needs more, nor does a prefill that runs unsplit.
     void *counters = nullptr;
@@ -1344,18 +1337,27 @@ int mslim_attn_record_payloads(void *ctx, void *k_pool, void *v_pool, int64_t po
     return check_hip(mslim::launch_record_payloads(l, direction == 0, c.stream), "record payload launch");
 }
 
-// The fp32 partials of a launch's split products (none when nothing is split),
-// in a context buffer that only grows (stage code 400 if it cannot).
-// `products`: sums per output, 2 for SwiGLU.
-static int proj_partials(Context &c, std::initializer_list<int> rows, int products, int inner, int tokens,
-                         float **partial) {
-    *partial = nullptr;
-    const size_t floats = mslim::proj_partial_floats(rows.begin(), (int)rows.size(), products, inner, tokens);
-    if (!floats) return 0;
-    if (grow_recorded(c, &c.proj_partial, &c.proj_partial_bytes, floats * sizeof(float), "hipMalloc projection partials"))
-        return 400;
-    *partial = static_cast<float *>(c.proj_partial);
-    return 0;
+// The plan of a launch of tiled products, and its fp32 partials in a context
+// buffer that only grows.  Where the buffer cannot be had, under capture above
+// all, the launch runs unsplit, to the same bits.
+struct Tiled {
+    mslim::ProjPlan plan;
+    float *partial;
+};
+static Tiled tiled_products(Context &c, const mslim::SkinnyMatrix *m, int count, const uint16_t *w_up,
+                            const uint16_t *x, int inner, int tokens) {
+    const mslim::ProjPlan plan = mslim::plan_proj(m, count, w_up, x, inner, tokens, true);
+    const size_t bytes = plan.partial_floats * sizeof(float);
+    if (c.proj_partial_bytes < bytes) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(c.stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone ||
+            grow_recorded(c, &c.proj_partial, &c.proj_partial_bytes, bytes, "hipMalloc projection partials")) {
+            (void)hipGetLastError();
+            g_error.clear();
+            return {mslim::plan_proj(m, count, w_up, x, inner, tokens, false), nullptr};
+        }
+    }
+    return {plan, static_cast<float *>(c.proj_partial)};
 }
 
 // One product on the context's stream: the MFMA decode kernel for up to 16
@@ -1369,9 +1371,8 @@ static int project(Context &c, const void *weight, const void *input, void *outp
         return check_hip(mslim::launch_skinny_gemm(&m, 1, x, inner, tokens, c.stream), "decode projection launch")
                    ? 404
                    : 0;
-    float *partial = nullptr;
-    if (int rc = proj_partials(c, {rows}, 1, inner, tokens, &partial)) return rc;
-    return check_hip(mslim::launch_proj(&m, 1, x, inner, tokens, partial, c.stream), "projection launch") ? 404 : 0;
+    const Tiled t = tiled_products(c, &m, 1, nullptr, x, inner, tokens);
+    return check_hip(mslim::launch_proj(t.plan, &m, 1, x, inner, tokens, t.partial, c.stream), "projection launch") ? 404 : 0;
 }
 
 // tv_hip_matrix_multiply's argument limits (hipblaslt_bridge.cpp:207-210).
@@ -1431,10 +1432,9 @@ int mslim_attn_gemm_bf16_add(void *ctx, const void *weight, const void *input, c
                    : 0;
     }
     const mslim::SkinnyMatrix m{w, static_cast<uint16_t *>(output), rows};
-    float *partial = nullptr;
-    if (int rc = proj_partials(c, {rows}, 1, inner, tokens, &partial)) return rc;
-    return check_hip(mslim::launch_proj_add(m, static_cast<const uint16_t *>(residual), x, inner, tokens, partial,
-                                            c.stream),
+    const Tiled t = tiled_products(c, &m, 1, nullptr, x, inner, tokens);
+    return check_hip(mslim::launch_proj_add(t.plan, m, static_cast<const uint16_t *>(residual), x, inner, tokens,
+                                            t.partial, c.stream),
                      "projection launch")
                ? 404
                : 0;
@@ -1459,12 +1459,11 @@ int mslim_attn_gemm_swiglu(void *ctx, const void *gate_weight, const void *up_we
                    ? 404
                    : 0;
     }
-    float *partial = nullptr;
-    if (int rc = proj_partials(c, {rows}, 2, inner, tokens, &partial)) return rc;
-    return check_hip(mslim::launch_proj_swiglu(static_cast<const uint16_t *>(gate_weight),
-                                               static_cast<const uint16_t *>(up_weight),
-                                               static_cast<uint16_t *>(output), rows, x, inner, tokens,
-                                               c.swiglu_table, partial, c.stream),
+    const auto *gw = static_cast<const uint16_t *>(gate_weight), *uw = static_cast<const uint16_t *>(up_weight);
+    const mslim::SkinnyMatrix m{gw, static_cast<uint16_t *>(output), rows};
+    const Tiled t = tiled_products(c, &m, 1, uw, x, inner, tokens);
+    return check_hip(mslim::launch_proj_swiglu(t.plan, m, uw, x, inner, tokens, c.swiglu_table, t.partial,
+                                               c.stream),
                      "projection launch")
                ? 404
                : 0;
@@ -1496,9 +1495,9 @@ int mslim_attn_gemm_qkv(void *ctx, const void *q_weight, const void *k_weight, c
         {static_cast<const uint16_t *>(q_weight), static_cast<uint16_t *>(q_out), q_rows},
         {static_cast<const uint16_t *>(k_weight), static_cast<uint16_t *>(k_out), kv_rows},
         {static_cast<const uint16_t *>(v_weight), static_cast<uint16_t *>(v_out), kv_rows}};
-    float *partial = nullptr;
-    if (int rc = proj_partials(c, {q_rows, kv_rows, kv_rows}, 1, inner, tokens, &partial)) return rc;
-    return check_hip(mslim::launch_proj(m, 3, static_cast<const uint16_t *>(input), inner, tokens, partial, c.stream),
+    const auto *x = static_cast<const uint16_t *>(input);
+    const Tiled t = tiled_products(c, m, 3, nullptr, x, inner, tokens);
+    return check_hip(mslim::launch_proj(t.plan, m, 3, x, inner, tokens, t.partial, c.stream),
                      "projection launch")
                ? 404
                : 0;
@@ -1570,9 +1569,9 @@ static int rmsnorm_gemm_qkv_locked(Context &c, const void *norm_weight, float ep
                          "decode projection launch")
                    ? 404
                    : 0;
-    float *partial = nullptr;
-    if (int rc = proj_partials(c, {q_rows, kv_rows, kv_rows}, 1, inner, tokens, &partial)) return rc;
-    return check_hip(mslim::launch_proj(m, 3, static_cast<const uint16_t *>(x), inner, tokens, partial, c.stream),
+    const Tiled t = tiled_products(c, m, 3, nullptr, static_cast<const uint16_t *>(x), inner, tokens);
+    return check_hip(mslim::launch_proj(t.plan, m, 3, static_cast<const uint16_t *>(x), inner, tokens, t.partial,
+                                        c.stream),
                      "projection launch")
                ? 404
                : 0;
@@ -1623,11 +1622,10 @@ int mslim_attn_rmsnorm_gemm_swiglu(void *ctx, const void *norm_weight, float eps
                          "decode projection launch")
                    ? 404
                    : 0;
-    float *partial = nullptr;
-    if (int rc = proj_partials(c, {rows}, 2, inner, tokens, &partial)) return rc;
-    return check_hip(mslim::launch_proj_swiglu(gw, uw, static_cast<uint16_t *>(output), rows,
-                                               static_cast<const uint16_t *>(x), inner, tokens, c.swiglu_table,
-                                               partial, c.stream),
+    const mslim::SkinnyMatrix m{gw, static_cast<uint16_t *>(output), rows};
+    const Tiled t = tiled_products(c, &m, 1, uw, static_cast<const uint16_t *>(x), inner, tokens);
+    return check_hip(mslim::launch_proj_swiglu(t.plan, m, uw, static_cast<const uint16_t *>(x), inner, tokens,
+                                               c.swiglu_table, t.partial, c.stream),
                      "projection launch")
                ? 404
                : 0;

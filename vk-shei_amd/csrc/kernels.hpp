@@ -301,20 +301,24 @@ hipError_t launch_skinny_swiglu(const uint16_t *w_gate, const uint16_t *w_up, ui
 // The same products for any number of token rows (csrc/proj.hip): the tiled
 // MFMA kernel when inner is a multiple of 64 and x and the weights are
 // 16-byte aligned, one wavefront per output otherwise.  Same epilogues.
-// Split launches keep fp32 partials in `partial`: proj_partial_floats floats
-// (0: not split), with products 2 for SwiGLU (gate and up) and 1 otherwise.
-size_t proj_partial_floats(const int *rows, int count, int products, int inner, int tokens);
-// Partials that every launch of inner < 8192 fits in: a context holds as much
-// from the start, so those launches never allocate.
-constexpr size_t kProjPartialBytes = (size_t)48 << 20;
-hipError_t launch_proj(const SkinnyMatrix *m, int count, const uint16_t *x, int inner, int tokens, float *partial,
-                       hipStream_t stream);
-hipError_t launch_proj_add(const SkinnyMatrix &m, const uint16_t *resid, const uint16_t *x, int inner, int tokens,
-                           float *partial, hipStream_t stream);
-// act_table: launch_swiglu_table's table (device, 128 KiB).
-hipError_t launch_proj_swiglu(const uint16_t *w_gate, const uint16_t *w_up, uint16_t *out, int rows,
-                              const uint16_t *x, int inner, int tokens, const uint16_t *act_table, float *partial,
-                              hipStream_t stream);
+// A plan says how a launch runs: its tile and which of its matrices are cut
+// along k; it changes no bit of the results.  A launch whose plan has
+// partial_floats keeps that many fp32 partials in `partial`; with may_split
+// false it has none.
+struct ProjPlan {
+    int tile;                        // -1: one wavefront per output
+    int ksegs[3];                    // segments of each matrix's sums, of the matrix alone
+    int ksplit[3];                   // 1, or ksegs: a workgroup per segment
+    size_t partial_floats;
+};
+ProjPlan plan_proj(const SkinnyMatrix *m, int count, const uint16_t *w_up, const uint16_t *x, int inner, int tokens,
+                   bool may_split);
+hipError_t launch_proj(const ProjPlan &plan, const SkinnyMatrix *m, int count, const uint16_t *x, int inner,
+                       int tokens, float *partial, hipStream_t stream);
+hipError_t launch_proj_add(const ProjPlan &plan, const SkinnyMatrix &m, const uint16_t *resid, const uint16_t *x,
+                           int inner, int tokens, float *partial, hipStream_t stream);
+hipError_t launch_proj_swiglu(const ProjPlan &plan, const SkinnyMatrix &gate, const uint16_t *w_up, const uint16_t *x,
+                              int inner, int tokens, const uint16_t *act_table, float *partial, hipStream_t stream);
 
 hipError_t launch_pages_write(uint16_t *k_pool, uint16_t *v_pool, const int32_t *page_table,
                               int page_tokens, int kv_heads, int head_dim, int64_t first_token,

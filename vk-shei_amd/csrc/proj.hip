@@ -17,9 +17,11 @@
 //   * fragment reads and copies are pinned between the MFMAs, and the last
 //     sub-step's MFMAs of a k-step run after the next barrier, behind the next
 //     stage's first fragment reads;
-//   * a product whose tiles would leave CUs idle is cut along k: each split
-//     writes fp32 partial sums and a second launch adds them in split order.
-//     The number of splits is a function of the product's shape alone;
+//   * the k range of a matrix is cut into segments, as many as its size alone
+//     says, each summed from zero and the sums added in order.  A launch whose
+//     tiles would leave CUs idle gives every segment a workgroup of its own
+//     that writes its fp32 sum, and a second launch adds them; any other
+//     launch adds them in registers, to the same bits;
 //   * tiles are dealt to XCDs in contiguous slices with the token tiles of a
 //     weight slice adjacent, so each weight row is read from HBM by one XCD;
 //   * epilogues: plain, residual add (out = BF16(resid + BF16(acc)), llm_add
@@ -27,8 +29,9 @@
 //     same tile (llm_swiglu after both), and up to three matrices with their
 //     own outputs in one launch (Q, K, V), each equal bit for bit to the
 //     plain product followed by the elementwise kernel.
-// Every split is summed by one wavefront in fixed k order, so results do not
-// depend on the tiling or on timing: a fused launch equals the separate ones.
+// Every segment is summed by one wavefront in fixed k order, so a token row's
+// results do not depend on the tiling, on the rows that share its launch (17 to
+// 512 of them) or on timing, and a fused launch equals the separate ones.
 // What bounds it: up to about 100 token rows the weights' HBM stream, above
 // them the latency of first reads (about 1.5 us against a ring of 64 to 96
 // KiB; the pure MFMA loop takes two thirds of the time at 512 tokens).
@@ -68,14 +71,16 @@ struct ProjArgs {
     const uint16_t *x;      // [tokens][inner]
     int inner, tokens;
     int n_tiles;            // token tiles
-    // Work items (row tile, token tile, k split) before segment s;
+    // Work items (row tile, token tile, k split) before matrix s;
     // [segments] = all.
     int first_item[kMaxSeg + 1];
-    // ksplit[s] > 1: item (tile, k split i) sums k-steps [i nk / ksplit,
-    // (i + 1) nk / ksplit) of segment s into partial + part_base[s], fp32
-    // [ksplit][product][tokens][rows], product the gate (0) or up (1) sum of
-    // SwiGLU; a second launch adds the partials in split order and applies
-    // the epilogue.
+    // Matrix s is summed in ksegs[s] segments of its k-steps [i nk / ksegs,
+    // (i + 1) nk / ksegs).  ksplit[s] is 1 (an item adds them all up) or
+    // ksegs[s] (item (tile, i) writes segment i to partial + part_base[s], fp32
+    // [ksegs][product][tokens][rows], product the gate (0) or up (1) sum of
+    // SwiGLU; a second launch adds the partials in order and applies the
+    // epilogue).
+    int ksegs[kMaxSeg];
     int ksplit[kMaxSeg];
     int64_t part_base[kMaxSeg];
     float *partial;
@@ -112,7 +117,10 @@ constexpr int proj_lds_bytes(int epi) {
     return table_in_lds<C>(epi) && stages < kTableBytes ? kTableBytes : stages;
 }
 
-template <class C, int EPI>
+// SUM: some item adds up several segments.  The totals and the test per k-step
+// would cost the launches without one 2% (gate and up of a 4,096 / 14,336 layer
+// at 17 to 64 tokens: 50.1 us, with them 51.2).
+template <class C, int EPI, bool SUM>
 __global__ __launch_bounds__(C::WAVES * 64) __attribute__((amdgpu_waves_per_eu(C::WAVES / 4))) void proj_kernel(ProjArgs a) {
     constexpr int kStages = C::ST;
     constexpr int kBM = C::BM;
@@ -167,6 +175,7 @@ __global__ __launch_bounds__(C::WAVES * 64) __attribute__((amdgpu_waves_per_eu(C
     const int nk_all = inner / kBK;
     const int kb = (int)((int64_t)split * nk_all / ksplit);
     const int nk = (int)((int64_t)(split + 1) * nk_all / ksplit) - kb;
+    const int ksegs = !SUM || ksplit > 1 ? 1 : s2 ? a.ksegs[2] : s1 ? a.ksegs[1] : a.ksegs[0];  // of this item
 
     // Copy offsets: chunk c of a stage is RPC rows; lane l lands in row
     // RPC c + l / NSL, physical slot l % NSL, and fetches the logical slot
@@ -238,6 +247,35 @@ __global__ __launch_bounds__(C::WAVES * 64) __attribute__((amdgpu_waves_per_eu(C
                 if (EPI == kSwiglu) accu[i][j][r] = 0.0f;
             }
 
+    // Sums of the segments that are complete.  -0 leaves the first one as it
+    // is, whatever its sign of zero.
+    floatx16_t total[MI][NJ], totalu[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                total[i][j][r] = -0.0f;
+                if (EPI == kSwiglu) totalu[i][j][r] = -0.0f;
+            }
+    auto end_segment = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    total[i][j][r] = __fadd_rn(total[i][j][r], acc[i][j][r]);
+                    acc[i][j][r] = 0.0f;
+                    if (EPI == kSwiglu) {
+                        totalu[i][j][r] = __fadd_rn(totalu[i][j][r], accu[i][j][r]);
+                        accu[i][j][r] = 0.0f;
+                    }
+                }
+    };
+    int seg = 1, seg_end = nk / ksegs;  // the first k-step after the current segment
+
     // Fragments of one sub-step: NJ of the tokens, MI of each weight matrix.
     struct Frag {
         bf16x8_t a[NA * MI], b[NJ];
@@ -307,6 +345,11 @@ __global__ __launch_bounds__(C::WAVES * 64) __attribute__((amdgpu_waves_per_eu(C
         raw_barrier();
         const int64_t k = k_bytes(kt + kStages - 1);
         phase(f1, f0, st, 0, mfma_tag, Yes{}, 0, sd, k);
+        if (SUM && kt == seg_end) {
+            end_segment();
+            ++seg;
+            seg_end = (int)((int64_t)seg * nk / ksegs);
+        }
 #pragma unroll
         for (int s = 0; s + 1 < SUB; ++s) {
             if (s % 2 == 0) phase(f0, f1, st, s + 1, Yes{}, Yes{}, s + 1, sd, k);
@@ -324,6 +367,7 @@ __global__ __launch_bounds__(C::WAVES * 64) __attribute__((amdgpu_waves_per_eu(C
         }
     }
     phase(f1, f0, 0, 0, Yes{}, No{}, SUB, 0, 0);
+    if (SUM) end_segment();
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // no copy may still target LDS at exit
 
     // SwiGLU: the activation table replaces the stages in LDS (one 128 KiB
@@ -342,6 +386,8 @@ __global__ __launch_bounds__(C::WAVES * 64) __attribute__((amdgpu_waves_per_eu(C
         table = reinterpret_cast<const uint16_t *>(lds);
     }
 
+    auto &sum = SUM ? total : acc;
+    auto &su = SUM ? totalu : accu;
     // Epilogue: lane l holds token WT wc + 32 j + l % 32 and, per group g of
     // four accumulators, rows WM wr + 32 i + 8 g + 4 h .. +3.
     if (ksplit > 1) {
@@ -361,20 +407,20 @@ __global__ __launch_bounds__(C::WAVES * 64) __attribute__((amdgpu_waves_per_eu(C
                     if (r >= rows) continue;
                     const int64_t o = (int64_t)t * rows + r;
                     if (vecf && r + 3 < rows) {
-                        const floatx4_t v = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2],
-                                             acc[i][j][4 * g + 3]};
+                        const floatx4_t v = {sum[i][j][4 * g], sum[i][j][4 * g + 1], sum[i][j][4 * g + 2],
+                                             sum[i][j][4 * g + 3]};
                         *reinterpret_cast<floatx4_t *>(part + o) = v;
                         if (EPI == kSwiglu) {
-                            const floatx4_t u = {accu[i][j][4 * g], accu[i][j][4 * g + 1], accu[i][j][4 * g + 2],
-                                                 accu[i][j][4 * g + 3]};
+                            const floatx4_t u = {su[i][j][4 * g], su[i][j][4 * g + 1], su[i][j][4 * g + 2],
+                                                 su[i][j][4 * g + 3]};
                             *reinterpret_cast<floatx4_t *>(part_up + o) = u;
                         }
                     } else {
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
                             if (r + e >= rows) break;
-                            part[o + e] = acc[i][j][4 * g + e];
-                            if (EPI == kSwiglu) part_up[o + e] = accu[i][j][4 * g + e];
+                            part[o + e] = sum[i][j][4 * g + e];
+                            if (EPI == kSwiglu) part_up[o + e] = su[i][j][4 * g + e];
                         }
                     }
                 }
@@ -396,8 +442,8 @@ __global__ __launch_bounds__(C::WAVES * 64) __attribute__((amdgpu_waves_per_eu(C
                 uint16_t y[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const uint16_t p = write_bf16(acc[i][j][4 * g + e]);
-                    if (EPI == kSwiglu) y[e] = swiglu_mul_bf16(table[p], write_bf16(accu[i][j][4 * g + e]));
+                    const uint16_t p = write_bf16(sum[i][j][4 * g + e]);
+                    if (EPI == kSwiglu) y[e] = swiglu_mul_bf16(table[p], write_bf16(su[i][j][4 * g + e]));
                     else y[e] = p;
                 }
                 const int64_t o = (int64_t)t * rows + r;
@@ -426,7 +472,7 @@ __global__ __launch_bounds__(C::WAVES * 64) __attribute__((amdgpu_waves_per_eu(C
     }
 }
 
-// Split segments (grid y): out = epilogue(BF16(partial[0] + partial[1] +
+// Split matrices (grid y): out = epilogue(BF16(partial[0] + partial[1] +
 // ...)), the partials added in split order, four outputs per thread.
 template <int EPI>
 __global__ __launch_bounds__(256) void proj_merge_kernel(ProjArgs a) {
@@ -561,98 +607,120 @@ constexpr double kStreamBytesPerUs = 4.8e6;   // weights from HBM
 constexpr double kMergeUs = 3.5;              // the merge launch, beside its traffic
 constexpr double kMergeBytesPerUs = 6.0e6;
 constexpr int kMinSplitSteps = 8;             // k-steps of a split, at least
-constexpr int64_t kSplitBytes = 16ll << 20;   // partials of one product's sum, at most (inner < 8192)
-constexpr double kGain = 0.5;                 // a larger tile or split must save this (us)
+constexpr int64_t kSplitBytes = 16ll << 20;   // partials of a launch, at most (inner < 8192; SwiGLU twice that)
+constexpr double kGain = 0.5;                 // a larger tile or a split must save this (us)
 
 int64_t tiles_of(const TileCost &c, int rows, int tokens) {
     return (int64_t)((rows + c.bm - 1) / c.bm) * ((tokens + c.bn - 1) / c.bn);
 }
 
-double split_cost(int ksplit, int64_t outputs) {
-    return ksplit == 1 ? 0.0 : kMergeUs + 2.0 * ksplit * outputs * sizeof(float) / kMergeBytesPerUs;
+// Partials of a split matrix, in whole 16-byte pieces.
+size_t split_floats(int ksplit, int products, int rows, int tokens) {
+    return ((size_t)ksplit * products * rows * tokens + 3) & ~(size_t)3;
 }
 
-// K splits of the product of a [rows][inner] matrix with `tokens` rows: the
-// count, on its best configuration, of the least predicted time.  It depends
-// on the product's own shape only, never on the launch the product is part
-// of, so every entry point (one matrix or several, fused epilogue or not) sums
-// a given product in the same order.  A narrow matrix counts as a square one:
-// it is a K or V beside its Q, whose splits leave the launch one wave of
-// workgroups, while splits of its own put more items behind them (Q, K, V of
-// 4,096 + 1,024 + 1,024 rows at 128 tokens: 20.9 us with Q's four splits for
-// all, 31.4 us with eight for K and V).
-int product_ksplit(int inner, int rows, int tokens) {
-    if (inner < 8192) rows = std::max(rows, std::min(inner, 4096));
-    const int steps = inner / kKAlign;
-    const double stream = (double)rows * inner * 2 / kStreamBytesPerUs;
-    const int64_t outputs = (int64_t)rows * tokens;
-    int best = 1;
-    double least = 0.0;
-    for (int k = 1; k <= 8; k *= 2) {
-        if (k > 1 && (steps / k < kMinSplitSteps ||
-                      (inner < 8192 && (int64_t)k * outputs * (int64_t)sizeof(float) > kSplitBytes)))
-            break;
-        double us = 0.0;
-        for (int t = 0; t < kTiles; ++t) {
-            const TileCost &c = kPlainCost[t];
-            const int64_t rounds = (tiles_of(c, rows, tokens) * k + kCus - 1) / kCus;
-            const double busy = rounds * ((steps + k - 1) / k) * c.step;
-            if (t == 0 || busy < us) us = busy;
-        }
-        us = std::max(us, stream) + split_cost(k, outputs);
-        if (k == 1 || us < least - kGain) {
-            least = us;
-            best = k;
-        }
-    }
-    return best;
-}
-
-// Configuration of a launch, given its products' splits: the one that
-// finishes first when its items are dealt to the resident workgroups.  Which
-// one it is changes no bit of the results.
-int choose_tile(const ProjArgs &a, bool swiglu) {
-    const int steps = a.inner / kKAlign;
-    int best = 0;
-    double least = 0.0;
-    for (int t = 0; t < kTiles; ++t) {
-        const TileCost &c = swiglu ? kSwigluCost[t] : kPlainCost[t];
-        int64_t items = 0;
-        double work = 0.0, longest = 0.0, bytes = 0.0;  // work and longest in k-steps
-        for (int s = 0; s < a.segments; ++s) {
-            const int64_t n = tiles_of(c, a.rows[s], a.tokens) * a.ksplit[s];
-            const double each = (double)steps / a.ksplit[s];
-            items += n;
-            work += n * each;
-            longest = std::max(longest, each);
-            bytes += (double)a.rows[s] * a.inner * 2 * (swiglu ? 2 : 1);
-        }
-        // equal items run in whole rounds; unequal ones leave about half of
-        // the longest item behind the mean
-        const double rounds = (double)((items + kCus - 1) / kCus);
-        const bool equal = work == items * longest;
-        const double span = equal ? rounds * longest : std::max(longest, work / kCus + (rounds > 1 ? longest / 2 : 0.0));
-        const double us = std::max(span * c.step, bytes / kStreamBytesPerUs);
-        if (t == 0 || us < least - kGain) {
-            least = us;
-            best = t;
-        }
-    }
-    return best;
+// Segments that a [rows][inner] matrix is summed in: as many as give every CU
+// about one 64 x 64 tile's segment, a power of two, eight k-steps at least.
+// From the matrix alone: a token row gets the same bits in every launch of more
+// than 16 rows, and K and V beside their Q those of a launch of their own.
+//   * 320 tiles' segments at most, since more queue behind one another (8,192
+//     rows and inputs at 64 tokens: 33 us with two, 45 with four); 640 from
+//     16,384 inputs, whose segments are long enough (28,672 inputs to 8,192
+//     rows: 64 tokens 107 us with two, 98 with four, 150 tokens 165 and 123).
+//   * One where there are more than twice as many rows as inputs (gate, up, the
+//     LM head): the sums are too short for a merge, and adding segments in
+//     registers is not free either (2,048 inputs to 8,192 rows at 300 tokens:
+//     31.2 us with one, 32.1 with two).
+//   * Eight only from 8,192 inputs and a quarter as many rows, the down
+//     projections: K and V of fewer rows share a launch with Q, and their
+//     eight splits put more items behind Q's (8,192 + 1,024 + 1,024 rows of
+//     8,192 inputs at 128 tokens: 107 us, with four at most 55).
+int k_segments(int inner, int rows) {
+    const int most = inner >= 8192 && (int64_t)rows * 4 >= inner ? 8 : 4;
+    const int64_t tiles = (rows + 63) / 64, limit = inner >= 16384 ? 640 : 320;
+    int n = 1;
+    if (rows > 2 * inner) return n;
+    while (n < most && tiles * n * 2 <= limit && inner / kKAlign / (n * 2) >= kMinSplitSteps) n *= 2;
+    return n;
 }
 
 }  // namespace
 
-size_t proj_partial_floats(const int *rows, int count, int products, int inner, int tokens) {
-    size_t total = 0;
-    for (int s = 0; s < count; ++s) {
-        const int k = product_ksplit(inner, rows[s], tokens);
-        if (k > 1) total += ((size_t)k * products * rows[s] * tokens + 3) & ~(size_t)3;
+// The choice that finishes first when the launch's items are dealt to the
+// resident workgroups and the merge, if any, is added.
+ProjPlan plan_proj(const SkinnyMatrix *m, int count, const uint16_t *w_up, const uint16_t *x, int inner, int tokens,
+                   bool may_split) {
+    ProjPlan best{};
+    bool fast = inner % kKAlign == 0 && aligned16(x) && (!w_up || aligned16(w_up));
+    for (int s = 0; s < count; ++s) fast = fast && aligned16(m[s].w);
+    best.tile = fast ? 0 : -1;
+    if (!fast) return best;
+    const int steps = inner / kKAlign, products = w_up ? 2 : 1;
+    for (int s = 0; s < count; ++s) best.ksegs[s] = k_segments(inner, m[s].rows);
+    // Unsplit, all matrices split, and of Q, K, V either Q or the others.
+    const int masks[4] = {0, 7, 1, 6};
+    double least = -1.0;
+    for (int k = 0; k < (may_split ? count == 3 ? 4 : 2 : 1); ++k) {
+        ProjPlan p = best;
+        p.partial_floats = 0;
+        double merge = 0.0;
+        for (int s = 0; s < count; ++s) {
+            p.ksplit[s] = masks[k] >> s & 1 ? p.ksegs[s] : 1;
+            if (p.ksplit[s] == 1) continue;
+            const size_t floats = split_floats(p.ksplit[s], products, m[s].rows, tokens);
+            p.partial_floats += floats;
+            merge += 2.0 * floats * sizeof(float) / kMergeBytesPerUs;
+        }
+        if (k && !p.partial_floats) continue;
+        // the merge's model is fitted up to here; past it 300 tokens of 4,096
+        // inputs and rows measured 30.1 us split, 25.1 unsplit
+        if (inner < 8192 && (int64_t)(p.partial_floats * sizeof(float)) > kSplitBytes * products) continue;
+        if (p.partial_floats) merge += kMergeUs;
+        for (p.tile = 0; p.tile < kTiles; ++p.tile) {
+            const TileCost &c = w_up ? kSwigluCost[p.tile] : kPlainCost[p.tile];
+            int64_t items = 0;
+            double work = 0.0, longest = 0.0, bytes = 0.0;  // work and longest in k-steps
+            for (int s = 0; s < count; ++s) {
+                const int64_t n = tiles_of(c, m[s].rows, tokens) * p.ksplit[s];
+                const double each = (double)steps / p.ksplit[s];
+                items += n;
+                work += n * each;
+                longest = std::max(longest, each);
+                bytes += (double)m[s].rows * inner * 2 * products;
+            }
+            // equal items run in whole rounds; unequal ones leave about half
+            // of the longest item behind the mean
+            const double rounds = (double)((items + kCus - 1) / kCus);
+            const bool equal = work == items * longest;
+            const double span =
+                equal ? rounds * longest : std::max(longest, work / kCus + (rounds > 1 ? longest / 2 : 0.0));
+            const double us = std::max(span * c.step, bytes / kStreamBytesPerUs) + merge;
+            if (least < 0.0 || us < least - kGain) {
+                least = us;
+                best = p;
+            }
+        }
     }
-    return total;
+    return best;
 }
 
 namespace {
+
+ProjArgs proj_args(const ProjPlan &plan, const SkinnyMatrix *m, int count, const uint16_t *x, int inner, int tokens) {
+    ProjArgs a{};
+    for (int s = 0; s < count; ++s) {
+        a.w[s] = m[s].w;
+        a.out[s] = m[s].out;
+        a.rows[s] = m[s].rows;
+        a.ksegs[s] = plan.ksegs[s];
+        a.ksplit[s] = plan.ksplit[s];
+    }
+    a.segments = count;
+    a.x = x;
+    a.inner = inner;
+    a.tokens = tokens;
+    return a;
+}
 
 template <class C, int EPI>
 hipError_t launch_config(ProjArgs &a, hipStream_t stream) {
@@ -662,32 +730,32 @@ hipError_t launch_config(ProjArgs &a, hipStream_t stream) {
         a.first_item[s + 1] = a.first_item[s] + (a.rows[s] + C::BM - 1) / C::BM * a.n_tiles * a.ksplit[s];
     for (int s = a.segments + 1; s <= kMaxSeg; ++s) a.first_item[s] = a.first_item[a.segments];
     const unsigned grid = (unsigned)((a.first_item[a.segments] + kXcds - 1) / kXcds * kXcds);
-    hipLaunchKernelGGL((proj_kernel<C, EPI>), dim3(grid), dim3(C::WAVES * 64), 0, stream, a);
+    bool sum = false;
+    for (int s = 0; s < a.segments; ++s) sum |= a.ksplit[s] < a.ksegs[s];
+    if (sum) hipLaunchKernelGGL((proj_kernel<C, EPI, true>), dim3(grid), dim3(C::WAVES * 64), 0, stream, a);
+    else hipLaunchKernelGGL((proj_kernel<C, EPI, false>), dim3(grid), dim3(C::WAVES * 64), 0, stream, a);
     return hipGetLastError();
 }
 
 template <int EPI>
-hipError_t launch(ProjArgs &a, hipStream_t stream) {
-    bool fast = a.inner % kKAlign == 0 && aligned16(a.x) && (EPI != kSwiglu || aligned16(a.w_up));
-    for (int s = 0; s < a.segments; ++s) fast = fast && aligned16(a.w[s]);
-    if (!fast) {
+hipError_t launch(const ProjPlan &plan, ProjArgs &a, float *partial, hipStream_t stream) {
+    if (plan.tile < 0) {
         int64_t total = 0;
         for (int s = 0; s < a.segments; ++s) total += (int64_t)a.rows[s] * a.tokens;
         hipLaunchKernelGGL((proj_generic_kernel<EPI>), dim3((unsigned)((total + 3) / 4)), dim3(256), 0, stream, a);
         return hipGetLastError();
     }
-    constexpr int products = EPI == kSwiglu ? 2 : 1;
+    if (plan.partial_floats && !partial) return hipErrorInvalidValue;
+    a.partial = partial;
     int64_t base = 0, most = 0;
     for (int s = 0; s < a.segments; ++s) {
-        a.ksplit[s] = product_ksplit(a.inner, a.rows[s], a.tokens);
         a.part_base[s] = base;
         if (a.ksplit[s] == 1) continue;
-        if (!a.partial) return hipErrorInvalidValue;
-        base += ((int64_t)a.ksplit[s] * products * a.rows[s] * a.tokens + 3) & ~(int64_t)3;
+        base += (int64_t)split_floats(a.ksplit[s], EPI == kSwiglu ? 2 : 1, a.rows[s], a.tokens);
         most = std::max(most, (int64_t)a.rows[s] * a.tokens);
     }
     hipError_t e;
-    switch (choose_tile(a, EPI == kSwiglu)) {
+    switch (plan.tile) {
         case kTile64x64: e = launch_config<TileConfig<kTile64x64, EPI>, EPI>(a, stream); break;
         case kTile64x128: e = launch_config<TileConfig<kTile64x128, EPI>, EPI>(a, stream); break;
         case kTile128x128: e = launch_config<TileConfig<kTile128x128, EPI>, EPI>(a, stream); break;
@@ -701,52 +769,25 @@ hipError_t launch(ProjArgs &a, hipStream_t stream) {
 
 }  // namespace
 
-hipError_t launch_proj(const SkinnyMatrix *m, int count, const uint16_t *x, int inner, int tokens, float *partial,
-                       hipStream_t stream) {
-    ProjArgs a{};
-    for (int s = 0; s < count; ++s) {
-        a.w[s] = m[s].w;
-        a.out[s] = m[s].out;
-        a.rows[s] = m[s].rows;
-    }
-    a.segments = count;
-    a.x = x;
-    a.inner = inner;
-    a.tokens = tokens;
-    a.partial = partial;
-    return launch<kPlain>(a, stream);
+hipError_t launch_proj(const ProjPlan &plan, const SkinnyMatrix *m, int count, const uint16_t *x, int inner,
+                       int tokens, float *partial, hipStream_t stream) {
+    ProjArgs a = proj_args(plan, m, count, x, inner, tokens);
+    return launch<kPlain>(plan, a, partial, stream);
 }
 
-hipError_t launch_proj_add(const SkinnyMatrix &m, const uint16_t *resid, const uint16_t *x, int inner, int tokens,
-                           float *partial, hipStream_t stream) {
-    ProjArgs a{};
-    a.w[0] = m.w;
-    a.out[0] = m.out;
-    a.rows[0] = m.rows;
-    a.segments = 1;
+hipError_t launch_proj_add(const ProjPlan &plan, const SkinnyMatrix &m, const uint16_t *resid, const uint16_t *x,
+                           int inner, int tokens, float *partial, hipStream_t stream) {
+    ProjArgs a = proj_args(plan, &m, 1, x, inner, tokens);
     a.resid = resid;
-    a.x = x;
-    a.inner = inner;
-    a.tokens = tokens;
-    a.partial = partial;
-    return launch<kAdd>(a, stream);
+    return launch<kAdd>(plan, a, partial, stream);
 }
 
-hipError_t launch_proj_swiglu(const uint16_t *w_gate, const uint16_t *w_up, uint16_t *out, int rows,
-                              const uint16_t *x, int inner, int tokens, const uint16_t *act_table, float *partial,
-                              hipStream_t stream) {
-    ProjArgs a{};
-    a.w[0] = w_gate;
+hipError_t launch_proj_swiglu(const ProjPlan &plan, const SkinnyMatrix &gate, const uint16_t *w_up, const uint16_t *x,
+                              int inner, int tokens, const uint16_t *act_table, float *partial, hipStream_t stream) {
+    ProjArgs a = proj_args(plan, &gate, 1, x, inner, tokens);
     a.w_up = w_up;
     a.act_table = act_table;
-    a.out[0] = out;
-    a.rows[0] = rows;
-    a.segments = 1;
-    a.x = x;
-    a.inner = inner;
-    a.tokens = tokens;
-    a.partial = partial;
-    return launch<kSwiglu>(a, stream);
+    return launch<kSwiglu>(plan, a, partial, stream);
 }
 
 }  // namespace mslim
