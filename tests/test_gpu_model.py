@@ -85,11 +85,12 @@ def test_argmax_bit_exact(ctx, rows, vocab):
     assert np.array_equal(out.cpu().numpy(), oracle.argmax_bf16(x, rows, vocab))
 
 
-@pytest.mark.parametrize("vocab", [8, 16, 8192, 8200, 131072, 131080, 140000, 8193])
+@pytest.mark.parametrize("vocab", [8, 16, 8192, 8200, 131072, 131080, 140000, 8193, 16384, 16392, 32768, 32776])
 def test_argmax_equal_values_over_chunks_and_lanes(ctx, vocab):
-    # A lane takes 8 logits a load, the workgroup 8,192, a full batch of loads
-    # 131,072: few distinct values, so that the first of many equal ones has to
-    # win within a chunk, a lane, a wavefront and across them.  Exact.
+    # A lane takes 8 logits a load, the workgroup 8,192, a batch of loads 1, 2, 4
+    # or (131,072) 16 times that: few distinct values, so that the first of many
+    # equal ones has to win within a chunk, a lane, a wavefront and across them.
+    # Exact.
     rng = np.random.default_rng(vocab)
     kinds = np.array([0.0, -0.0, -1.0, np.nan, -np.inf, -3.0], np.float32)
     rows = [rng.choice(kinds[a:], vocab) for a in (0, 1, 2, 3, 5)]

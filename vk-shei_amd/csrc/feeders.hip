@@ -422,12 +422,14 @@ __global__ __launch_bounds__(256) void embed_kernel(const uint16_t *table, const
 // decides.
 //
 // Bound by the lanes' comparisons, not by the row's bytes: one CU holds the
-// row.  VEC lanes (rows 16-byte aligned, vocab % 8 == 0) read 8 logits per
-// load with 16 loads in flight, which is a whole row of 131,072, keep only
+// row.  U > 0 (rows 16-byte aligned, vocab % 8 == 0): lanes read 8 logits per
+// load with U loads in flight, 16 of them a whole row of 131,072, keep only
 // the largest of the 8 and the chunk it came from (a comparison and a select
 // per logit, where tracking the index of each took eight instructions), and
 // one lane finds the logit in the winning chunk at the end.  A row of 128,256
-// logits: 13.2 us before, 6.8 us now; 20 rows 13.5 and 7.2.
+// logits: 13.2 us before, 6.8 us now; 20 rows 13.5 and 7.2.  Loads past a
+// row's end cost their comparisons too, so a short row takes the U that holds
+// it (32,000 logits: 6.8 us with 16, 4.5 with 4; 8,192: 6.9 and 4.5).
 constexpr int kArgmaxThreads = 1024;
 
 __device__ __forceinline__ void argmax_merge(float x, int i, float &best, int &index) {
@@ -437,7 +439,7 @@ __device__ __forceinline__ void argmax_merge(float x, int i, float &best, int &i
     }
 }
 
-template <bool VEC>
+template <int U>
 __global__ __launch_bounds__(kArgmaxThreads) void argmax_kernel(const uint16_t *logits, int rows, int vocab,
                                                                 int32_t *out) {
     __shared__ float values[kArgmaxThreads / 64];
@@ -447,10 +449,9 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_kernel(const uint16_t *
     const uint16_t *l = logits + (int64_t)row * vocab;
     const uint4 *l4 = reinterpret_cast<const uint4 *>(l);
     float best = -INFINITY;
-    int index = 0;  // VEC: of the chunk of 8
-    if (VEC) {
+    int index = 0;  // U > 0: of the chunk of 8
+    if constexpr (U > 0) {
         const int chunks = vocab / 8;
-        constexpr int U = 16;
         for (int base = tid; base < chunks; base += kArgmaxThreads * U) {
             uint4 v[U];
 #pragma unroll
@@ -495,7 +496,7 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_kernel(const uint16_t *
     if (tid != 0) return;
 #pragma unroll
     for (int w = 1; w < kArgmaxThreads / 64; ++w) argmax_merge(values[w], indices[w], best, index);
-    if (VEC) {
+    if constexpr (U > 0) {
         const uint4 v = l4[index];
         const uint32_t words[4] = {v.x, v.y, v.z, v.w};
         int at = 0;
@@ -725,12 +726,15 @@ hipError_t launch_embed(const uint16_t *table, const int32_t *ids, int tokens, i
 }
 
 hipError_t launch_argmax(const uint16_t *logits, int rows, int vocab, int32_t *out, hipStream_t stream) {
-    if (vocab % 8 == 0 && (reinterpret_cast<uintptr_t>(logits) & 15) == 0)
-        hipLaunchKernelGGL(argmax_kernel<true>, dim3((unsigned)rows), dim3(kArgmaxThreads), 0, stream, logits, rows,
-                           vocab, out);
-    else
-        hipLaunchKernelGGL(argmax_kernel<false>, dim3((unsigned)rows), dim3(kArgmaxThreads), 0, stream, logits, rows,
-                           vocab, out);
+    auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(kArgmaxThreads), 0, stream, logits, rows, vocab, out);
+    };
+    const int per_round = 8 * kArgmaxThreads;  // logits of one load per lane
+    if (vocab % 8 || (reinterpret_cast<uintptr_t>(logits) & 15)) run(argmax_kernel<0>);
+    else if (vocab <= per_round) run(argmax_kernel<1>);
+    else if (vocab <= 2 * per_round) run(argmax_kernel<2>);
+    else if (vocab <= 4 * per_round) run(argmax_kernel<4>);
+    else run(argmax_kernel<16>);
     return hipGetLastError();
 }
 
