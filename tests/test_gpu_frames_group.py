@@ -66,6 +66,12 @@ def test_group_kernel(ctx, qh, kvh, d, kf, vf, tokens):
         assert err <= bound, (shift, err, bound)
 
 
+@pytest.mark.parametrize("qh,kvh,d,tokens", [(2, 1, 8, 2048), (2, 1, 8, 2049), (16, 1, 16, 512), (16, 1, 16, 513)])
+def test_rows_of_few_pieces(ctx, qh, kvh, d, tokens):
+    # either side of the token count from which they take the group kernel
+    test_group_kernel(ctx, qh, kvh, d, F16, BF16, tokens)
+
+
 def test_group_kernel_ignores_what_follows_the_last_token(ctx):
     # rows past the token count hold infinities: lanes past the last token
     # must not read them into the result

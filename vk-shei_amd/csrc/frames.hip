@@ -576,8 +576,13 @@ hipError_t launch_value_format(const FramesArgs &a, int vf, bool grouped, bool v
 }  // namespace
 
 // Whole 16-byte pieces of K, V, Q and output rows (V and K rows of 8 elements
-// are 16 or 32 bytes) and a head dimension that 32 lanes hold.
+// are 16 or 32 bytes) and a head dimension that 32 lanes hold.  Rows of one or
+// two pieces leave most of their eight lanes idle, and over few tokens a token
+// per thread is faster (2/1 heads of 8: 256 tokens 4.9 us against 8.6, 2,000
+// tokens 8.7 and 9.7, 4,096 tokens 10.8 and 10.6; 16/1 heads of 16: 256 tokens
+// 6.2 and 8.5, 600 tokens 9.2 and 8.9).
 bool frames_grouped(const FramesLaunch &l) {
+    if (l.head_dim <= 16 && l.tokens * l.head_dim * l.head_dim <= 131072) return false;
     const uintptr_t p = reinterpret_cast<uintptr_t>(l.k) | reinterpret_cast<uintptr_t>(l.v) |
                         reinterpret_cast<uintptr_t>(l.q) | reinterpret_cast<uintptr_t>(l.out);
     return l.head_dim % 8 == 0 && l.head_dim <= 256 && (p & 15) == 0 && (int64_t)l.kv_heads * l.q_heads <= 65535;
