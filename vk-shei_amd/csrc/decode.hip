@@ -1025,7 +1025,7 @@ bool fixed_geometry(int head_dim, int group) {
 // buffers are aligned for its 16-byte loads (rows are: head_dim % 8 == 0) and
 // 8-byte stores; what is left runs one wavefront per query head.  Measured
 // (8 sequences of 500 .. 4,000 tokens, 24/8 heads of 128, 73 MB of K and V): 2,969 us with one
-// wavefront per query head, 19.3 us here.
+// wavefront per query head, 18.7 us here.
 bool decode_mfma(const DecodeLaunch &l) {
     const int group = l.q_heads / l.kv_heads;
     if (fixed_geometry(l.head_dim, group)) return true;

@@ -286,7 +286,7 @@ __device__ __forceinline__ float2 get_pair(const float *p) {
 // f32, as in frames_split_kernel, with exp2 of scores in log2 units.  Bound by
 // latency: the few loads each workgroup makes, then the count and the merge.  Against one workgroup per
 // (query head, split), whose lanes each walked a row of their own: 4,096
-// tokens of binary16, 32/8 heads of 128 (17 MB): 55.3 us (two launches) -> 12.9
+// tokens of binary16, 32/8 heads of 128 (17 MB): 55.3 us (two launches) -> 12.8
 // us; 300 tokens of 24/8 heads 8.0 us.
 // Loads of K, and of V, in flight per wavefront: four, two where eight heads'
 // queries and sums leave no registers for more.

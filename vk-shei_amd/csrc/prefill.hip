@@ -885,7 +885,7 @@ int row_block_tiles(const PrefillLaunch &l, int rows_per_block, int rb) {
 // Launches the MFMA kernel takes: head_dim 64 or 128, for the groups of its
 // WIDE form with buffers aligned for the 16-byte loads and 8-byte stores; what
 // is left runs one wavefront per query row and head.  Measured (1,001 queries
-// of 24/8 heads of 128): 5,523 us with a wavefront per row and head, 30.1 us
+// of 24/8 heads of 128): 5,523 us with a wavefront per row and head, 30.4 us
 // here.
 bool prefill_mfma(const PrefillLaunch &l) {
     if (l.head_dim != 64 && l.head_dim != 128) return false;
@@ -909,7 +909,8 @@ namespace {
 // chunk (the merge loads every other chunk's O as one uncached batch).  Fitted
 // to every chunk length measured on 28 launches of 256 to 3,072 queries after
 // 0 to 3,584 tokens, 4 to 8 heads per kv head: the chunk it picks is the
-// fastest measured or within 3.5% of it.
+// fastest measured or within 3.5% of it.  The WIDE form uses the same two
+// constants; its chunk lengths were not swept.
 constexpr double kItemFixedTiles = 7.0;
 constexpr double kMergeChunkTiles = 4.0;
 
