@@ -656,8 +656,13 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
             const uint16_t *kp = z.k + (int64_t)kvh * D, *vp = z.v + (int64_t)kvh * D + half * 4;
             auto score = [&](int t) __attribute__((always_inline)) {
                 float dot = 0.0f;
-#pragma unroll 1
-                for (int d = 0; d < D; ++d) dot = fmaf(read_bf16(qp[d]), read_bf16(kp[t * stride + d]), dot);
+#pragma unroll 2
+                for (int d = 0; d < D; d += 8) {
+                    const bf16x8_t qv = *reinterpret_cast<const bf16x8_t *>(qp + d);
+                    const bf16x8_t kv = *reinterpret_cast<const bf16x8_t *>(kp + t * stride + d);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) dot = fmaf((float)qv[e], (float)kv[e], dot);
+                }
                 return dot;
             };
             float m = -INFINITY;
@@ -671,14 +676,21 @@ __global__ __launch_bounds__(512, 1) void prefill_mfma_kernel(PrefillArgs a) {
                 for (int r = 0; r < 16; ++r) o[mt][r] = 0.0f;
 #pragma unroll 1
             for (int t = first_key; t < past_key; ++t) {
-                const float x = score(t);
-                const float p = x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(fmaf(x, z.scale_log2e, -m_used));
+                const float dot = score(t);
+                const float p = dot == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(fmaf(dot, z.scale_log2e, -m_used));
                 l += p;
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        o[mt][r] = fmaf(p, read_bf16(vp[t * stride + mt * 32 + r / 4 * 8 + r % 4]), o[mt][r]);
+                    for (int r4 = 0; r4 < 4; ++r4) {
+                        const uint2 w = *reinterpret_cast<const uint2 *>(vp + t * stride + mt * 32 + r4 * 8);
+                        const uint32_t two[2] = {w.x, w.y};
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float x = read_bf16((uint16_t)(two[e / 2] >> (e % 2 * 16)));
+                            o[mt][r4 * 4 + e] = fmaf(p, x, o[mt][r4 * 4 + e]);
+                        }
+                    }
             }
         }
     }
